@@ -9,13 +9,6 @@
 // The table must be the fp32 one the reference's loader produces
 // (reconstruct.py:52-62), so the bits match eptq.reconstruct.
 //
-// Layout: a thread takes (Q-row m, 8 consecutive columns) items with a
-// grid stride (consecutive threads, consecutive column chunks of one row):
-// one 16-byte index load and 16-byte g and h loads, and one 16-byte store in
-// each of the 8 output rows.  Workgroups stay resident and stage the E8-D4
-// table in LDS once.  The kernel is write-bound (16 bytes out per 2-byte
-// index).
-
 #include "common.h"
 #include "kernels.h"
 
@@ -31,62 +24,91 @@ __device__ __forceinline__ int csr_lower_bound(const int32_t* __restrict__ col,
   return lo;
 }
 
-constexpr int kDqPerCu = 16;  // resident workgroups per CU (8: ~3% slower on the 11008-wide layers)
+// One wave per (Q-row, 512 columns): every lane takes 8 columns (one 16-byte
+// index load, one 16-byte store in each of the 8 output rows), and the row's
+// critical blocks are found by the wave together.  The row's CSR entries are
+// in ascending column order, so the entry of a marker is the number of
+// entries left of the segment plus the number of markers before it in the
+// segment (ballots); its O vector comes from the lane that loaded it
+// (bpermute).  Rows of up to 64 entries load columns and vectors at once with
+// the indices, so a marker costs no memory round trip of its own; longer rows
+// count their entries left of the segment first.  An entry whose column does
+// not match (inconsistent CSR data) falls back to the search by column.
+//
+// Bound by the W writes (16 bytes out per 2-byte index).  Measured at 1% critical
+// blocks, 11008x4096: 41.1 -> 19.5 us (4.6 TB/s of W; a device copy moves 5.1,
+// a fill 6.9), 4096x4096: 17.3 -> 9.0 us, against one search by column per
+// marker and lane (nearly every wave held one); S_group 14336x4096 at 0.2%:
+// 89 -> 24 us (scale rows in 16-byte loads rather than one load per element).
+// 2, 8 and 64 workgroups per CU are within 3% of 4; more waves per SIMD through
+// fewer registers 20-100% slower; cached in place of streaming stores 18-36%
+// slower.
+constexpr int kSegCols = 512;
+constexpr int kSegWaves = 8;   // waves per workgroup: one 8 KB table fill per 64 KB or more of W
+constexpr int kSegPerCu = 4;   // workgroups per CU (2 resident at this register count, the rest follow)
 
 template <int KIND, bool HAS_S>
-__global__ __launch_bounds__(256) void k_dequant(
-    const int16_t* __restrict__ Q, const float* __restrict__ table,
-    const f16* __restrict__ g, const f16* __restrict__ h,
-    const f16* __restrict__ O, const int32_t* __restrict__ O_col,
-    const int32_t* __restrict__ O_row_ptr, const f16* __restrict__ S, int qb,
-    int M, int N, int chunks_per_row, int vec, f16* __restrict__ W) {
+__global__ __launch_bounds__(64 * kSegWaves) void k_dequant_seg(DequantArgs a, int segs, int tasks) {
   __shared__ f32x4 tab[KIND == KIND_E8D4 ? 512 : 1];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int N = a.N;
   if (KIND == KIND_E8D4) {
-    for (int i = threadIdx.x; i < 512; i += 256) tab[i] = ((const f32x4*)table)[i];
+    tab[threadIdx.x] = ((const f32x4*)a.table)[threadIdx.x];
+    static_assert(64 * kSegWaves == 512, "one table row per thread");
     __syncthreads();
   }
-  const int64_t items = (int64_t)M * chunks_per_row;
-  const int64_t stride = (int64_t)gridDim.x * 256;
-  // 16-byte path: the next item's index, g and h chunks are requested before
-  // the current item is computed (one item in flight per thread).
-  u16x8 qnext = {};
-  f16x8 hnext = {}, gnext = {};
-  auto fetch = [&](int64_t i) {
-    if (vec && i < items) {
-      const int mm = (int)(i / chunks_per_row);
-      const int nn = (int)(i - (int64_t)mm * chunks_per_row) * 8;
-      qnext = *(const u16x8*)(Q + (size_t)mm * N + nn);
-      hnext = *(const f16x8*)(h + nn);
-      gnext = *(const f16x8*)(g + 8 * mm);
+  for (int t = (int)blockIdx.x * kSegWaves + wave; t < tasks; t += (int)gridDim.x * kSegWaves) {
+    const int m = t / segs;
+    const int s0 = (t - m * segs) * kSegCols;   // the segment's first column
+    const int n0 = s0 + 8 * lane;
+    const bool act = n0 < N;                    // N % 8 == 0: whole chunks
+    const int r0 = a.O ? a.O_row_ptr[m] : 0, r1 = a.O ? a.O_row_ptr[m + 1] : 0;
+    u16x8 qv = {};
+    f16x8 hv = {}, sv = {};
+    if (act) {
+      qv = *(const u16x8*)(a.Q + (size_t)m * N + n0);
+      hv = *(const f16x8*)(a.h + n0);
+      if (HAS_S) sv = *(const f16x8*)(a.S + (size_t)(8 * m / a.qb) * N + n0);
     }
-  };
-  fetch((int64_t)blockIdx.x * 256 + threadIdx.x);
-  for (int64_t it = (int64_t)blockIdx.x * 256 + threadIdx.x; it < items; it += stride) {
-    const int m = (int)(it / chunks_per_row);
-    const int n0 = (int)(it - (int64_t)m * chunks_per_row) * 8;
-    // 16-byte accesses when the host found N % 8 == 0 and Q, g, h, W 16-byte
-    // aligned (every chunk then is whole); element by element otherwise.
-    const bool full = vec && n0 + 8 <= N;
-    const int r0 = O_row_ptr[m], r1 = O_row_ptr[m + 1];
+    // The row's entries, one per lane: all of them here, or (more than 64)
+    // those from the segment's first one on, below.
+    int ecol = 0x7fffffff;
+    u32x4 eo = {};
+    auto load_entries = [&](int first) {
+      if (first + lane < r1) {
+        ecol = a.O_col[first + lane];
+        eo = *(const u32x4*)(a.O + (size_t)(first + lane) * 8);
+      }
+    };
+    const bool whole = r1 - r0 <= 64;
+    if (whole) load_entries(r0);
     float gk[8];
-    int16_t q8[8];
-    f16 h8[8];
-    if (vec) {
 #pragma unroll
-      for (int c = 0; c < 8; ++c) {
-        gk[c] = (float)gnext[c];
-        q8[c] = (int16_t)qnext[c];
-        h8[c] = hnext[c];
+    for (int k = 0; k < 8; ++k) gk[k] = (float)a.g[8 * m + k];
+
+    uint64_t mk[8], any = 0;
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      mk[c] = __ballot(qv[c] == 0x7fffu);
+      any |= mk[c];
+    }
+    int src = 0;   // the lane that holds the entry of this lane's next marker
+    if (any) {
+      if (whole) {
+        src = __popcll(__ballot(ecol < s0));
+      } else {
+        int first = r0;
+        for (int e = r0; e < r1; e += 64) {
+          const int left = __popcll(__ballot(e + lane < r1 && a.O_col[e + lane < r1 ? e + lane : r1 - 1] < s0));
+          first += left;
+          if (left < 64) break;
+        }
+        load_entries(first);
       }
-      fetch(it + stride);
-    } else {
 #pragma unroll
-      for (int k = 0; k < 8; ++k) gk[k] = (float)g[8 * m + k];
-#pragma unroll
-      for (int c = 0; c < 8; ++c) {
-        q8[c] = n0 + c < N ? Q[(size_t)m * N + n0 + c] : (int16_t)0;
-        h8[c] = n0 + c < N ? h[n0 + c] : (f16)0.0f;
-      }
+      for (int c = 0; c < 8; ++c)
+        src = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mk[c] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mk[c], src));
     }
     // out[k] word c/2: the fp16 pair (column c, column c + 1) of output row
     // 8m + k, converted two at a time (one v_cvt_pk_f16_f32).
@@ -96,33 +118,49 @@ __global__ __launch_bounds__(256) void k_dequant(
       float v[2][8];
 #pragma unroll
       for (int cc = 0; cc < 2; ++cc) {
-        const int n = n0 + c + cc;
-        const unsigned u = (unsigned)((int)q8[c + cc] + 32768);
-        if (u == 65535u) {
-          const int i = csr_lower_bound(O_col, r0, r1, n);
-          const bool hit = (i < r1) && (O_col[i] == n);
-#pragma unroll
-          for (int k = 0; k < 8; ++k) v[cc][k] = hit ? (float)O[(size_t)i * 8 + k] : 0.0f;
+        unsigned u = (unsigned)qv[c + cc] ^ 0x8000u;   // index + 32768; 65535 marks a critical block
+        f32x4 lo, hi;
+        if (KIND == KIND_E8D4) {
+          lo = tab[u >> 7];
+          hi = tab[((u >> 14) << 7) | (u & 127u)];
         } else {
-          f32x4 a, b;
-          if (KIND == KIND_E8D4) {
-            a = tab[u >> 7];
-            b = tab[((u >> 14) << 7) | (u & 127u)];
-          } else {
-            const f32x4* p = (const f32x4*)(table + (size_t)u * 8);
-            a = p[0];
-            b = p[1];
-          }
-          v[cc][0] = a.x; v[cc][1] = a.y; v[cc][2] = a.z; v[cc][3] = a.w;
-          v[cc][4] = b.x; v[cc][5] = b.y; v[cc][6] = b.z; v[cc][7] = b.w;
-          if (HAS_S) {
+          u = u == 65535u ? 0u : u;   // past the table
+          const f32x4* p = (const f32x4*)(a.table + (size_t)u * 8);
+          lo = p[0];
+          hi = p[1];
+        }
 #pragma unroll
-            for (int k = 0; k < 8; ++k)
-              v[cc][k] = n < N ? v[cc][k] * (float)S[(size_t)((8 * m + k) / qb) * N + n] : v[cc][k];
+        for (int k = 0; k < 4; ++k) {
+          v[cc][k] = lo[k];
+          v[cc][k + 4] = hi[k];
+        }
+        if (HAS_S) {
+          const float s = (float)sv[c + cc];
+#pragma unroll
+          for (int k = 0; k < 8; ++k) v[cc][k] *= s;
+        }
+        if (mk[c + cc]) {   // uniform
+          const bool mine = qv[c + cc] == 0x7fffu;
+          const int n = n0 + c + cc;
+          u32x4 o;
+#pragma unroll
+          for (int d = 0; d < 4; ++d) o[d] = (uint32_t)__builtin_amdgcn_ds_bpermute(4 * src, (int)eo[d]);
+          const int oc = __builtin_amdgcn_ds_bpermute(4 * src, ecol);
+          const bool found = src < 64 && oc == n;
+          if (mine) {
+            if (!found) {   // inconsistent data, or over 64 markers in the segment
+              const int i = csr_lower_bound(a.O_col, r0, r1, n);
+              const bool hit = i < r1 && a.O_col[i] == n;
+              o = hit ? *(const u32x4*)(a.O + (size_t)i * 8) : u32x4{};
+            }
+            const f16x8 of = __builtin_bit_cast(f16x8, o);
+#pragma unroll
+            for (int k = 0; k < 8; ++k) v[cc][k] = (float)of[k];
+            ++src;
           }
         }
       }
-      const float h0 = (float)h8[c], h1 = (float)h8[c + 1];
+      const float h0 = (float)hv[c], h1 = (float)hv[c + 1];
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
         float w0 = (v[0][k] * gk[k]) * h0;
@@ -134,18 +172,63 @@ __global__ __launch_bounds__(256) void k_dequant(
         out[k][c >> 1] = __builtin_bit_cast(uint32_t, (f16x2){(f16)w0, (f16)w1});
       }
     }
+    if (act) {
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      f16* dst = W + (size_t)(8 * m + k) * N + n0;
-      if (full) {
-        __builtin_nontemporal_store(out[k], (u32x4*)dst);   // streamed out, not re-read here
+      for (int k = 0; k < 8; ++k)
+        __builtin_nontemporal_store(out[k], (u32x4*)(a.W + (size_t)(8 * m + k) * N + n0));   // not re-read here
+    }
+  }
+}
+
+// Element by element, for column counts or pointers that rule the 16-byte
+// accesses out: a thread takes (Q-row, 8 columns) items with a grid stride.
+constexpr int kDqPerCu = 16;  // resident workgroups per CU
+
+template <int KIND, bool HAS_S>
+__global__ __launch_bounds__(256) void k_dequant(DequantArgs a, int chunks_per_row) {
+  __shared__ f32x4 tab[KIND == KIND_E8D4 ? 512 : 1];
+  if (KIND == KIND_E8D4) {
+    for (int i = threadIdx.x; i < 512; i += 256) tab[i] = ((const f32x4*)a.table)[i];
+    __syncthreads();
+  }
+  const int M = a.M, N = a.N;
+  const int64_t items = (int64_t)M * chunks_per_row;
+  const int64_t stride = (int64_t)gridDim.x * 256;
+  for (int64_t it = (int64_t)blockIdx.x * 256 + threadIdx.x; it < items; it += stride) {
+    const int m = (int)(it / chunks_per_row);
+    const int n0 = (int)(it - (int64_t)m * chunks_per_row) * 8;
+    const int r0 = a.O_row_ptr[m], r1 = a.O_row_ptr[m + 1];
+    for (int n = n0; n < N && n < n0 + 8; ++n) {
+      const unsigned u = (unsigned)((int)a.Q[(size_t)m * N + n] + 32768);
+      float v[8];
+      if (u == 65535u) {
+        const int i = csr_lower_bound(a.O_col, r0, r1, n);
+        const bool hit = (i < r1) && (a.O_col[i] == n);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[k] = hit ? (float)a.O[(size_t)i * 8 + k] : 0.0f;
       } else {
-        for (int c = 0; c < 8 && n0 + c < N; ++c) {
-          // Through a local: this compiler's __builtin_bit_cast of a vector
-          // element lvalue reads element 0.
-          const uint32_t wd = out[k][c >> 1];
-          dst[c] = __builtin_bit_cast(f16x2, wd)[c & 1];
+        f32x4 lo, hi;
+        if (KIND == KIND_E8D4) {
+          lo = tab[u >> 7];
+          hi = tab[((u >> 14) << 7) | (u & 127u)];
+        } else {
+          const f32x4* p = (const f32x4*)(a.table + (size_t)u * 8);
+          lo = p[0];
+          hi = p[1];
         }
+        const float s = HAS_S ? (float)a.S[(size_t)(8 * m / a.qb) * N + n] : 1.0f;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          v[k] = HAS_S ? lo[k] * s : lo[k];
+          v[k + 4] = HAS_S ? hi[k] * s : hi[k];
+        }
+      }
+      const float hn = (float)a.h[n];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        float w = (v[k] * (float)a.g[8 * m + k]) * hn;
+        asm volatile("" : "+v"(w));   // two roundings, as above
+        a.W[(size_t)(8 * m + k) * N + n] = (f16)w;
       }
     }
   }
@@ -153,21 +236,26 @@ __global__ __launch_bounds__(256) void k_dequant(
 
 template <int KIND>
 int launch_dequant(const DequantArgs& a, hipStream_t s) {
-  const int chunks = (a.N + 7) / 8;
-  const int64_t items = (int64_t)a.M * chunks;
   int dev = 0, cus = 256;
   if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-  const int vec = (a.N % 8 == 0) &&
-                  ((((uintptr_t)a.Q | (uintptr_t)a.g | (uintptr_t)a.h | (uintptr_t)a.W) & 15u) == 0);
-  int64_t blocks = (items + 255) / 256;
+  // 16-byte accesses: whole 8-column chunks, every operand they touch aligned.
+  const bool vec = a.N % 8 == 0 &&
+                   ((((uintptr_t)a.Q | (uintptr_t)a.h | (uintptr_t)a.W | (uintptr_t)a.S | (uintptr_t)a.O) & 15u) == 0);
+  const int segs = (a.N + kSegCols - 1) / kSegCols;
+  const int64_t tasks = (int64_t)a.M * segs;
+  if (vec && tasks <= 0x3fffffff) {
+    int64_t blocks = (tasks + kSegWaves - 1) / kSegWaves;
+    if (blocks > (int64_t)cus * kSegPerCu) blocks = (int64_t)cus * kSegPerCu;
+    if (a.S) k_dequant_seg<KIND, true><<<(unsigned)blocks, 64 * kSegWaves, 0, s>>>(a, segs, (int)tasks);
+    else k_dequant_seg<KIND, false><<<(unsigned)blocks, 64 * kSegWaves, 0, s>>>(a, segs, (int)tasks);
+    return 0;
+  }
+  const int chunks = (a.N + 7) / 8;
+  int64_t blocks = ((int64_t)a.M * chunks + 255) / 256;
   if (blocks > (int64_t)cus * kDqPerCu) blocks = (int64_t)cus * kDqPerCu;
   if (blocks < 1) return 0;
-  if (a.S)
-    k_dequant<KIND, true><<<(unsigned)blocks, 256, 0, s>>>(
-        a.Q, a.table, a.g, a.h, a.O, a.O_col, a.O_row_ptr, a.S, a.qb, a.M, a.N, chunks, vec, a.W);
-  else
-    k_dequant<KIND, false><<<(unsigned)blocks, 256, 0, s>>>(
-        a.Q, a.table, a.g, a.h, a.O, a.O_col, a.O_row_ptr, nullptr, 1, a.M, a.N, chunks, vec, a.W);
+  if (a.S) k_dequant<KIND, true><<<(unsigned)blocks, 256, 0, s>>>(a, chunks);
+  else k_dequant<KIND, false><<<(unsigned)blocks, 256, 0, s>>>(a, chunks);
   return 0;
 }
 

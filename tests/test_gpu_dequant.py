@@ -79,3 +79,24 @@ def test_dequant_markers_first_last_column_and_full_rows():
     for kind, r in (("e8_d4", 1.75), ("e8_lattice", 1.6)):
         W, ref = _run(kind, r, qd)
         _assert_bits(W, ref)
+
+
+@pytest.mark.parametrize("kind,radius", [("e8_d4", 1.75), ("e8_lattice", 1.6)])
+@pytest.mark.parametrize("N", [8, 504, 512, 520, 1536, 2056])
+def test_dequant_markers_over_512_column_segments(kind, radius, N):
+    """Bit equality where a wave's 512-column segment ends, rows hold 0, 1, 64, 65 or all columns as critical blocks,
+    or more than 64 fall into one segment."""
+    print(f"dequant segments {kind} N={N}", flush=True)
+    qd = make_layer(128, N, seed=N, percmask=0.0, qb_size=64)
+    rng = np.random.default_rng(N)
+    Q = qd.Q.clone()
+    for m, count in enumerate([0, 1, 63, 64, 65, 70, 128, N, N // 2, 0, 1, 200, 64, N, 3, 65]):
+        Q[m, torch.from_numpy(rng.permutation(N)[:min(count, N)].copy())] = 32767
+    if N > 512:
+        Q[9, 505:512], Q[9, 512:519] = 32767, 32767
+    qd.Q = Q
+    qd.O = torch.from_numpy(rng.standard_normal((int((Q == 32767).sum()), 8)).astype(np.float16))
+    for S in (qd.S_group, None):
+        qd.S_group = S
+        W, ref = _run(kind, radius, qd)
+        _assert_bits(W, ref)
