@@ -1393,19 +1393,8 @@ size_t static_lds(const void* kern) {
 
 template <int KIND>
 int launch_gemm(const LinearArgs& a, hipStream_t s, void* work, long long work_bytes) {
-  if (KIND == KIND_E8D4 && a.B <= kSliceMaxTokens && a.prep == 0) {
-    // Eligibility does not depend on the slice (B = 1..16 all qualify), so a
-    // first slice that launches means every slice does.
-    int rc = 0;
-    for (int b0 = 0; b0 < a.B && rc == 0; b0 += kMatvecMaxBatch) {
-      LinearArgs t = a;
-      t.B = a.B - b0 < kMatvecMaxBatch ? a.B - b0 : kMatvecMaxBatch;
-      t.x = a.x + (size_t)b0 * a.ldx;
-      t.y = a.y + (size_t)b0 * a.ldy;
-      rc = launch_decode_mfma_multi(&t, 1, s);
-    }
-    if (rc == 0) return 0;
-  }
+  if (KIND == KIND_E8D4 && a.B <= kWideMaxTokens && launch_decode_wide_multi(&a, 1, s, work, work_bytes) == 0)
+    return 0;
   // LDS-decode kernel: fp16 x and table, no S_group, K-steps of 64, whole
   // 8-, 16-, 20- or 32-Q-row tiles, 16-byte x rows and 8-byte y stores.  Of the two
   // tile widths, the one with less work per CU (rounds of the CUs × tile

@@ -111,6 +111,11 @@ int launch_decode_e8d4_pair(const LinearArgs* layers, hipStream_t s);
 // silu(gate) ⊙ up with the roundings of the separate SwiGLU kernel.
 int launch_decode_mfma_multi(const LinearArgs* layers, int n, hipStream_t s, void* work = nullptr,
                              long long work_bytes = 0, uint16_t* act = nullptr);
+// Matrix-core E8-D4 decode for up to kWideMaxTokens rows, each index decoded
+// once for up to 64 of them (fp16 or bf16 x, fp16 table, no prep, no
+// residual); -1 when the layers are outside its range.
+int launch_decode_wide_multi(const LinearArgs* layers, int n, hipStream_t s, void* work = nullptr,
+                             long long work_bytes = 0);
 // Split-K workspace of the matrix-core decode kernel: kSplitCounters int
 // arrival counters (one per 64-row tile of a launch), then fp32 partial sums,
 // kSplitPartBytes per (split tile, part): [16 batch rows][64 outputs], then
@@ -136,13 +141,7 @@ inline int mfma_min_batch() {
 
 // Largest batch served by the decode matvec; larger batches take the GEMM.
 constexpr int kMatvecMaxBatch = 16;
-// Up to this many rows an E8-D4 launch runs as 16-row slices of the
-// matrix-core decode kernel: its 64-row tiles spread a layer over far more
-// workgroups than the GEMM's 128-token tiles can at these token counts (one
-// token tile: 32 workgroups for 4096 rows), and the slices re-read the weight
-// from cache.  Measured at 32 / 128 / 256 tokens on 4096x4096: slices 27 /
-// 106 / 214 us against 112 us for the GEMM; 4096x11008: 59 / 226 / 459 us
-// against 285-290 us.
-constexpr int kSliceMaxTokens = 128;
+// Up to this many rows an E8-D4 launch runs on the wide matrix-core decode.
+constexpr int kWideMaxTokens = 128;
 
 }  // namespace eptq

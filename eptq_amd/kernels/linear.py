@@ -15,7 +15,7 @@ Differences, all towards the reference's own reconstruct semantics:
 * ``S_group`` layers stay compressed and run the fused grouped kernel instead
   of a materialized fp16 W (``kernels/linear.py:97-120,158-164``).
 * every batch size runs a hand-written HIP kernel of this library: the decode
-  matvec for ≤16 rows, 16-row slices of the matrix-core decode up to 128 rows,
+  matvec for ≤16 rows, the wide matrix-core decode (E8-D4) up to 128 rows,
   the prefill GEMM that decodes weight tiles into LDS above (the reference's
   ``csrc/eptq_kernels.cu:520-537`` route), and from 2048 fp16 tokens (256
   for S_group layers or bf16 x, 64 for E8 layers) the two-pass prefill: each weight

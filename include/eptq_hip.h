@@ -94,13 +94,13 @@ typedef struct {
  *
  * work: NULL, or a 16-byte aligned device buffer of work_bytes bytes,
  * zero-filled before its first use (eptq_e8d4_work_bytes() bytes cover every
- * launch).  With it, batches (or 16-row slices) of 3..16 rows on layers with
- * few 64-row tiles have each tile's columns split over up to 4 workgroups,
+ * launch).  With it, batches of 3..128 rows on layers with few 64-row tiles
+ * have each tile's columns split over up to 4 workgroups (8 from 17 rows),
  * whose fp32 partial sums meet in the buffer (the kernel leaves its counters
  * at zero), and prefill launches above 128 rows whose tiles leave half the
  * CUs idle or more split K over up to 4 parts whose fp32 sums a second launch
- * adds in part order (a 64 MiB area past the decode part; a smaller buffer
- * only takes the decode split).  Calls that share a buffer must not run at
+ * adds in part order (a 64 MiB area past the decode part, which 17..128 rows
+ * use too; a smaller buffer splits less).  Calls that share a buffer must not run at
  * the same time.
  */
 int eptq_e8d4_forward_multi(int n_layers, const eptq_layer* layers, const void* codes,
