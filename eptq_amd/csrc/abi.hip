@@ -160,7 +160,7 @@ int linear_common(int kind, const void* Q, const void* codes, int codes_dtype, c
 int dequant_common(int kind, const void* Q, const void* codes_f32, const void* g,
                    const void* h, const void* O_vals, const void* O_col,
                    const void* O_row_ptr, const void* S_group, int n_groups, int M, int N,
-                   void* W, void* stream) {
+                   void* W, void* stream, int keep = 0, int table_f16 = 0) {
   const char* fn = kind == eptq::KIND_E8D4 ? "eptq_e8d4_dequant" : "eptq_e8_dequant";
   int qb = 1;
   int rc = check_common(fn, Q, codes_f32, g, h, O_vals, O_col, O_row_ptr, S_group, n_groups, M,
@@ -172,7 +172,7 @@ int dequant_common(int kind, const void* Q, const void* codes_f32, const void* g
     return fail(EPTQ_EUNSUPPORTED, "%s: W must be 8-byte aligned", fn);
   eptq::DequantArgs a;
   a.Q = (const int16_t*)Q;
-  a.table = (const float*)codes_f32;
+  a.table = codes_f32;
   a.g = (const eptq::f16*)g;
   a.h = (const eptq::f16*)h;
   a.O = (const eptq::f16*)O_vals;
@@ -183,6 +183,8 @@ int dequant_common(int kind, const void* Q, const void* codes_f32, const void* g
   a.M = M;
   a.N = N;
   a.W = (eptq::f16*)W;
+  a.keep = keep;
+  a.table_f16 = table_f16;
   hipStream_t s = (hipStream_t)stream;
   rc = kind == eptq::KIND_E8D4 ? eptq::launch_dequant<eptq::KIND_E8D4>(a, s)
                                : eptq::launch_dequant<eptq::KIND_E8>(a, s);
@@ -477,8 +479,10 @@ int eptq_f16_gemm_rows(const void* W, const void* x, const void* bias, int F, in
   if (ranges_overlap(y, y_bytes, x, (size_t)T * N * 2) || ranges_overlap(y, y_bytes, W, (size_t)F * N * 2) ||
       ranges_overlap(y, y_bytes, row_scale, (size_t)T * 4))
     return fail(EPTQ_EINVAL, "%s: y overlaps x, W or row_scale", fn);
-  if (eptq::launch_gemm_f16w((const uint16_t*)W, (const uint16_t*)x, (const eptq::f16*)bias, F, N, T, N, (uint16_t*)y,
-                             ldy, (hipStream_t)stream, (const float*)row_scale, y_dtype == EPTQ_BF16) != 0)
+  const eptq::f16* b = (const eptq::f16*)bias;
+  const int start = 0;
+  if (eptq::launch_gemm_f16w((const uint16_t*)W, (const uint16_t*)x, 1, &b, &start, F, N, T, N, (uint16_t*)y, ldy,
+                             (hipStream_t)stream, (const float*)row_scale, y_dtype == EPTQ_BF16) != 0)
     return fail(EPTQ_EUNSUPPORTED, "%s: F=%d N=%d ldy=%d (multiples of 64, 64, 4) or alignment", fn, F, N, ldy);
   return check_launch(fn);
 }
@@ -500,6 +504,166 @@ int eptq_bf16_rows_to_f16(const void* x, int N, int T, void* x16, void* row_scal
   if (eptq::launch_bf16_rows_to_f16((const uint16_t*)x, N, T, (uint16_t*)x16, (float*)row_scale,
                                     (hipStream_t)stream) != 0)
     return fail(EPTQ_EUNSUPPORTED, "%s: N=%d (a multiple of 8 up to 16384) or alignment", fn, N);
+  return check_launch(fn);
+}
+
+// The two-pass prefill's estimated time, and whether its layers run together
+// (all W in one buffer, one GEMM: few-row layers, grouped-query k and v,
+// leave CUs idle alone) or one after another.  The constants (the dequantizer
+// at 4.4 TB/s with W kept in the caches, keep_w, and 5 past them, after which
+// the GEMM takes 10% longer; 2.5 us per launch, 9 more per fused launch than
+// its steps) choose between the two forms, over the 108 measured pairs of
+// Llama-2-7B, 13B and Llama-3-8B units at 129 to 2048 rows, within 0.6% of the
+// faster one on average.
+struct TwoPass {
+  bool together;
+  double us;
+};
+static bool keep_w(double bytes) { return bytes <= 160e6; }   // the last-level cache holds 256 MB
+static TwoPass plan_two_pass(int n, const eptq_layer* layers, int N, int B, size_t room) {
+  double apart = 0.0;
+  long long F = 0;
+  auto gemm = [&](long long f, double bytes) {
+    return eptq::f16w_estimate_us((int)f, N, B, room) * (keep_w(bytes) ? 1.0 : 1.1);
+  };
+  for (int l = 0; l < n; ++l) {
+    const double bytes = 16.0 * layers[l].M * N;
+    F += 8LL * layers[l].M;
+    apart += gemm(8LL * layers[l].M, bytes) + bytes / (keep_w(bytes) ? 4.4e6 : 5.0e6) + 5.0;
+  }
+  if (n < 2 || n > eptq::kMaxLayers || F > 0x7fffffff) return {false, apart};
+  const double bytes = 2.0 * F * N;
+  const double all = gemm(F, bytes) + bytes / (keep_w(bytes) ? 4.4e6 : 5.0e6) + 2.5 * n + 2.5;
+  return all < 0.97 * apart ? TwoPass{true, all} : TwoPass{false, apart};
+}
+
+static size_t split_room(const void* work, long long work_bytes) {
+  const long long off = eptq::decode_mfma_work_bytes();
+  return work && work_bytes > off ? (size_t)(work_bytes - off) : 0;
+}
+
+static bool two_pass_shape(int n_layers, const eptq_layer* layers, int N, int B, int x_dtype) {
+  if (n_layers < 1 || !layers || N <= 0 || N % 64 != 0 || B < 1) return false;
+  if (x_dtype != EPTQ_F16 && (x_dtype != EPTQ_BF16 || N > 16384)) return false;   // bf16 rows to fp16
+  for (int l = 0; l < n_layers; ++l)
+    if (layers[l].M <= 0 || layers[l].M % 8 != 0 || layers[l].M > 0x7fffffff / 64) return false;
+  return true;
+}
+
+// Scratch of a call: W, then for bf16 x its fp16 rows and their scales.
+struct TwoPassScratch {
+  long long w, x16, rs, bytes;
+};
+static TwoPassScratch two_pass_scratch(long long w, int N, int B, int x_dtype) {
+  auto up = [](long long v) { return (v + 255) / 256 * 256; };
+  const bool bf = x_dtype == EPTQ_BF16;
+  const long long x16 = up(w), rs = x16 + (bf ? up(2LL * B * N) : 0);
+  return {w, x16, rs, rs + (bf ? 4LL * B : 0)};
+}
+static void two_pass_w(int n, const eptq_layer* layers, int N, long long* sum, long long* most) {
+  *sum = *most = 0;
+  for (int l = 0; l < n; ++l) {
+    const long long b = 16LL * layers[l].M * N;
+    *sum += b;
+    *most = b > *most ? b : *most;
+  }
+}
+
+static bool two_pass_preferred(bool e8, int n_layers, const eptq_layer* layers, int N, int B, int x_dtype, size_t room) {
+  if (B <= eptq::kMatvecMaxBatch) return false;
+  if (e8) return true;
+  if (B <= eptq::kWideMaxTokens) return false;
+  bool all_s = true;
+  for (int l = 0; l < n_layers; ++l) all_s = all_s && layers[l].S_group;
+  if (x_dtype != EPTQ_F16 || all_s) return true;
+  double fused = 0.0;
+  for (int l = 0; l < n_layers; ++l) {
+    const double us = layers[l].S_group ? -1.0 : eptq::fused_estimate_us(layers[l].M, N, B, room);
+    if (us < 0.0) return true;
+    fused += us + 9.0;
+  }
+  return plan_two_pass(n_layers, layers, N, B, room).us < fused;
+}
+
+long long eptq_two_pass_scratch_bytes(int e8, int n_layers, const eptq_layer* layers, int N, int B, int x_dtype,
+                                      int has_work, int always) {
+  if (!two_pass_shape(n_layers, layers, N, B, x_dtype)) return 0;
+  const size_t room = has_work ? eptq::kPrefillSplitBytes : 0;
+  if (!always && !two_pass_preferred(e8 != 0, n_layers, layers, N, B, x_dtype, room)) return 0;
+  long long sum, most;
+  two_pass_w(n_layers, layers, N, &sum, &most);
+  return two_pass_scratch(plan_two_pass(n_layers, layers, N, B, room).together ? sum : most, N, B, x_dtype).bytes;
+}
+
+int eptq_two_pass_forward(int e8, int n_layers, const eptq_layer* layers, const void* codes, int codes_dtype,
+                          const void* x, int x_dtype, int N, int B, void* y, int ldy, void* scratch,
+                          long long scratch_bytes, void* work, long long work_bytes, void* stream) {
+  const char* fn = "eptq_two_pass_forward";
+  const int kind = e8 ? eptq::KIND_E8 : eptq::KIND_E8D4;
+  if (n_layers < 1 || !layers) return fail(EPTQ_EINVAL, "%s: n_layers=%d", fn, n_layers);
+  if (N <= 0 || B < 0) return fail(EPTQ_EINVAL, "%s: N=%d B=%d", fn, N, B);
+  if (x_dtype != EPTQ_F16 && x_dtype != EPTQ_BF16)
+    return fail(EPTQ_EINVAL, "%s: x_dtype must be EPTQ_F16 or EPTQ_BF16", fn);
+  if (codes_dtype != EPTQ_F16 && codes_dtype != EPTQ_F32)
+    return fail(EPTQ_EINVAL, "%s: codes_dtype must be EPTQ_F16 or EPTQ_F32", fn);
+  if (B == 0) return EPTQ_OK;
+  if (!x || !y || !scratch || !codes) return fail(EPTQ_EINVAL, "%s: null x/y/scratch/codes", fn);
+  if (work && (!aligned16(work) || work_bytes < 0))
+    return fail(EPTQ_EINVAL, "%s: work must be 16-byte aligned with work_bytes >= 0", fn);
+  if (!two_pass_shape(n_layers, layers, N, B, x_dtype))
+    return fail(EPTQ_EUNSUPPORTED, "%s: N=%d (a multiple of 64; up to 16384 for bf16 x), M of every layer a multiple of 8", fn, N);
+  if (!aligned16(x) || ((uintptr_t)scratch & 255) != 0 || ldy % 4 != 0 || ((uintptr_t)y & 7) != 0)
+    return fail(EPTQ_EUNSUPPORTED, "%s: ldy=%d (a multiple of 4) or alignment", fn, ldy);
+  long long at = 0, sum, most;
+  bool packed = true;   // outputs side by side from column 0
+  for (int l = 0; l < n_layers; ++l) {
+    const eptq_layer& L = layers[l];
+    if (((uintptr_t)L.bias & 7) != 0) return fail(EPTQ_EUNSUPPORTED, "%s: layer %d: bias alignment", fn, l);
+    if (L.y_offset < 0 || L.y_offset + 8LL * L.M > (long long)ldy || (L.y_offset & 3))
+      return fail(EPTQ_EINVAL, "%s: layer %d columns [%lld, %lld) outside a y row of %d (offset %% 4 == 0)", fn, l,
+                  L.y_offset, L.y_offset + 8LL * L.M, ldy);
+    packed = packed && L.y_offset == at;
+    at += 8LL * L.M;
+  }
+  two_pass_w(n_layers, layers, N, &sum, &most);
+  const TwoPassScratch least = two_pass_scratch(most, N, B, x_dtype), full = two_pass_scratch(sum, N, B, x_dtype);
+  if (scratch_bytes < least.bytes)
+    return fail(EPTQ_EINVAL, "%s: scratch of %lld bytes, %lld needed", fn, scratch_bytes, least.bytes);
+  const size_t x_bytes = (size_t)B * N * 2, y_bytes = (size_t)B * ldy * 2;
+  if (ranges_overlap(scratch, (size_t)scratch_bytes, x, x_bytes) || ranges_overlap(y, y_bytes, x, x_bytes) ||
+      ranges_overlap(y, y_bytes, scratch, (size_t)scratch_bytes))
+    return fail(EPTQ_EINVAL, "%s: x, y and scratch must not overlap", fn);
+  hipStream_t s = (hipStream_t)stream;
+  const bool all = packed && scratch_bytes >= full.bytes &&
+                   plan_two_pass(n_layers, layers, N, B, split_room(work, work_bytes)).together;
+  const TwoPassScratch& sc = all ? full : least;
+  uint16_t* const W = (uint16_t*)scratch;
+  const uint16_t* xg = (const uint16_t*)x;
+  const float* rs = nullptr;
+  if (x_dtype == EPTQ_BF16) {
+    uint16_t* x16 = (uint16_t*)((char*)scratch + sc.x16);
+    float* r = (float*)((char*)scratch + sc.rs);
+    if (eptq::launch_bf16_rows_to_f16(xg, N, B, x16, r, s) != 0) return fail(EPTQ_EUNSUPPORTED, "%s: N=%d", fn, N);
+    xg = x16;
+    rs = r;
+  }
+  const eptq::f16* biases[eptq::kMaxLayers];
+  int starts[eptq::kMaxLayers], pending = 0, F = 0;
+  for (int l = 0; l < n_layers; ++l) {
+    const eptq_layer& L = layers[l];
+    if (const int rc = dequant_common(kind, L.Q, codes, L.g, L.h, L.O_vals, L.O_col, L.O_row_ptr, L.S_group,
+                                      L.n_groups, L.M, N, W + (size_t)F * N, stream,
+                                      keep_w(all ? (double)sum : 16.0 * L.M * N), codes_dtype == EPTQ_F16))
+      return rc;
+    biases[pending] = (const eptq::f16*)L.bias;
+    starts[pending++] = F;
+    F += 8 * L.M;
+    if (all && l + 1 < n_layers) continue;
+    if (eptq::launch_gemm_f16w(W, xg, pending, biases, starts, F, N, B, N, (uint16_t*)y + (all ? 0 : L.y_offset), ldy,
+                               s, rs, x_dtype == EPTQ_BF16, work, work ? work_bytes : 0) != 0)
+      return fail(EPTQ_EUNSUPPORTED, "%s: F=%d N=%d ldy=%d", fn, F, N, ldy);
+    pending = F = 0;
+  }
   return check_launch(fn);
 }
 

@@ -42,7 +42,8 @@ __device__ __forceinline__ int csr_lower_bound(const int32_t* __restrict__ col,
 // 89 -> 24 us (scale rows in 16-byte loads rather than one load per element).
 // 2, 8 and 64 workgroups per CU are within 3% of 4; more waves per SIMD through
 // fewer registers 20-100% slower; cached in place of streaming stores 18-36%
-// slower.
+// slower, but a GEMM that reads W next finds part of it in the last-level
+// cache: both passes of 13824x5120 at 2048 tokens 298 -> 280 us (keep).
 constexpr int kSegCols = 512;
 constexpr int kSegWaves = 8;   // waves per workgroup: one 8 KB table fill per 64 KB or more of W
 constexpr int kSegPerCu = 4;   // workgroups per CU (2 resident at this register count, the rest follow)
@@ -54,7 +55,12 @@ __global__ __launch_bounds__(64 * kSegWaves) void k_dequant_seg(DequantArgs a, i
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int N = a.N;
   if (KIND == KIND_E8D4) {
-    tab[threadIdx.x] = ((const f32x4*)a.table)[threadIdx.x];
+    if (a.table_f16) {   // uniform
+      const f16x4 v = ((const f16x4*)a.table)[threadIdx.x];
+      tab[threadIdx.x] = (f32x4){(float)v[0], (float)v[1], (float)v[2], (float)v[3]};
+    } else {
+      tab[threadIdx.x] = ((const f32x4*)a.table)[threadIdx.x];
+    }
     static_assert(64 * kSegWaves == 512, "one table row per thread");
     __syncthreads();
   }
@@ -125,9 +131,15 @@ __global__ __launch_bounds__(64 * kSegWaves) void k_dequant_seg(DequantArgs a, i
           hi = tab[((u >> 14) << 7) | (u & 127u)];
         } else {
           u = u == 65535u ? 0u : u;   // past the table
-          const f32x4* p = (const f32x4*)(a.table + (size_t)u * 8);
-          lo = p[0];
-          hi = p[1];
+          if (a.table_f16) {          // uniform
+            const f16x8 v = ((const f16x8*)a.table)[u];
+            lo = (f32x4){(float)v[0], (float)v[1], (float)v[2], (float)v[3]};
+            hi = (f32x4){(float)v[4], (float)v[5], (float)v[6], (float)v[7]};
+          } else {
+            const f32x4* p = (const f32x4*)a.table + (size_t)u * 2;
+            lo = p[0];
+            hi = p[1];
+          }
         }
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
@@ -174,8 +186,11 @@ __global__ __launch_bounds__(64 * kSegWaves) void k_dequant_seg(DequantArgs a, i
     }
     if (act) {
 #pragma unroll
-      for (int k = 0; k < 8; ++k)
-        __builtin_nontemporal_store(out[k], (u32x4*)(a.W + (size_t)(8 * m + k) * N + n0));   // not re-read here
+      for (int k = 0; k < 8; ++k) {
+        u32x4* dst = (u32x4*)(a.W + (size_t)(8 * m + k) * N + n0);
+        if (a.keep) *dst = out[k];                       // uniform
+        else __builtin_nontemporal_store(out[k], dst);   // not re-read here
+      }
     }
   }
 }
@@ -187,8 +202,13 @@ constexpr int kDqPerCu = 16;  // resident workgroups per CU
 template <int KIND, bool HAS_S>
 __global__ __launch_bounds__(256) void k_dequant(DequantArgs a, int chunks_per_row) {
   __shared__ f32x4 tab[KIND == KIND_E8D4 ? 512 : 1];
+  auto row4 = [&](size_t r) {   // four table values
+    if (!a.table_f16) return ((const f32x4*)a.table)[r];
+    const f16x4 v = ((const f16x4*)a.table)[r];
+    return (f32x4){(float)v[0], (float)v[1], (float)v[2], (float)v[3]};
+  };
   if (KIND == KIND_E8D4) {
-    for (int i = threadIdx.x; i < 512; i += 256) tab[i] = ((const f32x4*)a.table)[i];
+    for (int i = threadIdx.x; i < 512; i += 256) tab[i] = row4(i);
     __syncthreads();
   }
   const int M = a.M, N = a.N;
@@ -212,9 +232,8 @@ __global__ __launch_bounds__(256) void k_dequant(DequantArgs a, int chunks_per_r
           lo = tab[u >> 7];
           hi = tab[((u >> 14) << 7) | (u & 127u)];
         } else {
-          const f32x4* p = (const f32x4*)(a.table + (size_t)u * 8);
-          lo = p[0];
-          hi = p[1];
+          lo = row4(2 * (size_t)u);
+          hi = row4(2 * (size_t)u + 1);
         }
         const float s = HAS_S ? (float)a.S[(size_t)(8 * m / a.qb) * N + n] : 1.0f;
 #pragma unroll

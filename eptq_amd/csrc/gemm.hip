@@ -1007,6 +1007,43 @@ __global__ __launch_bounds__(64 * (8 + NPW), (8 + NPW) / 4) void k_gemm_lds_e8d4
   }
 }
 
+// Bias of up to kMaxLayers layers side by side (null: none); a layer starts at
+// a multiple of 8 features.
+struct BiasCols {
+  const f16* b[kMaxLayers];
+  int start[kMaxLayers];   // first feature of each layer, past F for unused ones
+  __device__ __forceinline__ f16x4 at(int f) const {
+    const f16* p = b[0];
+    int s = 0;
+#pragma unroll
+    for (int l = 1; l < kMaxLayers; ++l)
+      if (f >= start[l]) {
+        p = b[l];
+        s = start[l];
+      }
+    return p ? *(const f16x4*)(p + (f - s)) : f16x4{};
+  }
+};
+
+// K split of a W-streaming GEMM: tiles [0, T1) take one workgroup each, the
+// others P, whose fp32 sums [part][tile - T1][token][feature] a second launch
+// adds.  Workgroups are dealt to the 8 XCDs round-robin: each XCD gets a run
+// of consecutive tiles.
+struct KSplit {
+  int tiles, T1, P;
+  float* part;
+  struct Unit { int tile, part, P, tail; };
+  __device__ __forceinline__ static int deal(int b, int n) { return (n & 7) == 0 ? (b & 7) * (n >> 3) + (b >> 3) : b; }
+  __device__ __forceinline__ Unit unit(int b, int grid) const {
+    if (b < T1) return {deal(b, T1), 0, 1, 0};
+    const int u = deal(b - T1, grid - T1), tail = tiles - T1;
+    return {T1 + u % tail, u / tail, P, tail};
+  }
+  __device__ __forceinline__ float* at(const Unit& u, int tile_floats) const {
+    return part + ((size_t)u.part * u.tail + (u.tile - T1)) * tile_floats;
+  }
+};
+
 // Four outputs of one token: y = acc · sc + bias, rounded to fp16 or (ybf)
 // bf16; sc is the token's power-of-two activation scale (1 for fp16 x).
 __device__ __forceinline__ void store_out(uint16_t* p, const f32x4& acc, float sc, const f16x4& b4, int ybf) {
@@ -1034,8 +1071,9 @@ __device__ __forceinline__ void store_out(uint16_t* p, const f32x4& acc, float s
 // rest; F is a multiple of BF here, rs and ybf as in k_gemm_f16w4.
 template <int BF, int NPW, int NS, int GT = 4>
 __global__ __launch_bounds__(64 * (8 + NPW), (8 + NPW) / 4) void k_gemm_f16w(
-    const uint16_t* __restrict__ W, const uint16_t* __restrict__ x, const f16* __restrict__ bias, int N, int T,
-    int ldx, uint16_t* __restrict__ y, int ldy, int OB, int F, const float* __restrict__ rs, int ybf) {
+    const uint16_t* __restrict__ W, const uint16_t* __restrict__ x, BiasCols bias, int N, int T, int ldx,
+    uint16_t* __restrict__ y, int ldy, int OB, int F, const float* __restrict__ rs, int ybf,
+    KSplit sp) {
   constexpr int kBK = g3::kBK, kBT = g3::kBT;
   constexpr int XS = kBT * 128, WS = BF * 128, W0 = NS * XS;
   static_assert(NS == 2 || NS == 3, "stages");
@@ -1045,21 +1083,19 @@ __global__ __launch_bounds__(64 * (8 + NPW), (8 + NPW) / 4) void k_gemm_f16w(
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // Workgroups are dealt to the 8 XCDs round-robin: give each XCD a run of
-  // consecutive tiles (same token tile, neighbouring feature tiles).
-  int blk = blockIdx.x;
-  const int G = gridDim.x;
-  if ((G & 7) == 0) blk = (blk & 7) * (G >> 3) + (blk >> 3);
   // Tiles in bands of GT token tiles, token tile fastest: the 32 consecutive
   // tiles one XCD runs at a time cover GT token tiles x 32/GT feature tiles,
   // so each x and W slice comes from the last-level cache once per XCD and
   // from the XCD's L2 for the rest.
-  const int TBn = G / OB;
-  const int band = blk / (GT * OB), r = blk - band * GT * OB;
+  const KSplit::Unit un = sp.unit(blockIdx.x, gridDim.x);
+  const int TBn = sp.tiles / OB;
+  const int band = un.tile / (GT * OB), r = un.tile - band * GT * OB;
   const int gt = min(GT, TBn - band * GT);
   const int ob = r / gt, tb = band * GT + r % gt;
   const int f0 = ob * BF, t0 = tb * kBT;
-  const int nk = N / kBK;
+  const int k0 = un.part * (N / kBK) / un.P, nk = (un.part + 1) * (N / kBK) / un.P - k0;
+  W += k0 * kBK;
+  x += k0 * kBK;
 
   if (wave >= 8) {
     // ================= producer waves 8 .. 8 + NPW - 1 =================
@@ -1157,13 +1193,13 @@ __global__ __launch_bounds__(64 * (8 + NPW), (8 + NPW) / 4) void k_gemm_f16w(
 #pragma unroll
   for (int xx = 0; xx < FA; ++xx) {
     const int f = f0 + wf * FW + 16 * xx + 4 * kg;
-    f16x4 b4 = {};
-    if (bias) b4 = *(const f16x4*)(bias + f);
+    const f16x4 b4 = bias.at(f);
 #pragma unroll
     for (int q = 0; q < TB; ++q) {
       const int tt = t0 + wt * TW + 16 * q + i;
       if (tt >= T) continue;
-      store_out(y + (size_t)tt * ldy + f, acc[xx][q], rs ? rs[tt] : 1.0f, b4, ybf);
+      if (un.P > 1) *(f32x4*)(sp.at(un, kBT * BF) + (tt - t0) * BF + (f - f0)) = acc[xx][q];
+      else store_out(y + (size_t)tt * ldy + f, acc[xx][q], rs ? rs[tt] : 1.0f, b4, ybf);
     }
   }
 }
@@ -1182,8 +1218,9 @@ __global__ __launch_bounds__(64 * (8 + NPW), (8 + NPW) / 4) void k_gemm_f16w(
 // the output is rs[t] · acc + bias in fp16 or (ybf) bf16.
 template <int BF, int BT, int GT = 4>
 __global__ __launch_bounds__(512, 2) void k_gemm_f16w4(
-    const uint16_t* __restrict__ W, const uint16_t* __restrict__ x, const f16* __restrict__ bias, int N, int T,
-    int ldx, uint16_t* __restrict__ y, int ldy, int OB, int F, const float* __restrict__ rs, int ybf) {
+    const uint16_t* __restrict__ W, const uint16_t* __restrict__ x, BiasCols bias, int N, int T, int ldx,
+    uint16_t* __restrict__ y, int ldy, int OB, int F, const float* __restrict__ rs, int ybf,
+    KSplit sp) {
   constexpr int kBK = g3::kBK, kBT = BT, NS = 3, NPW = 4;
   constexpr int XS = kBT * 128, WS = BF * 128, W0 = NS * XS;
   constexpr int FW = BF / 2, FA = FW / 16, TW = kBT / 2, TB = TW / 16;
@@ -1192,16 +1229,15 @@ __global__ __launch_bounds__(512, 2) void k_gemm_f16w4(
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  int blk = blockIdx.x;
-  const int G = gridDim.x;
-  if ((G & 7) == 0) blk = (blk & 7) * (G >> 3) + (blk >> 3);
-  // Tiles in bands of GT token tiles, token tile fastest (as k_gemm_f16w).
-  const int TBn = G / OB;
-  const int band = blk / (GT * OB), r = blk - band * GT * OB;
+  const KSplit::Unit un = sp.unit(blockIdx.x, gridDim.x);   // bands of GT token tiles (as k_gemm_f16w)
+  const int TBn = sp.tiles / OB;
+  const int band = un.tile / (GT * OB), r = un.tile - band * GT * OB;
   const int gt = min(GT, TBn - band * GT);
   const int ob = r / gt, tb = band * GT + r % gt;
   const int f0 = ob * BF, t0 = tb * kBT;
-  const int nk = N / kBK;
+  const int k0 = un.part * (N / kBK) / un.P, nk = (un.part + 1) * (N / kBK) / un.P - k0;
+  W += k0 * kBK;
+  x += k0 * kBK;
 
   if (wave >= 4) {
     // ================= producer waves 4 .. 7 =================
@@ -1329,13 +1365,13 @@ __global__ __launch_bounds__(512, 2) void k_gemm_f16w4(
   for (int xx = 0; xx < FA; ++xx) {
     const int f = f0 + wf * FW + 16 * xx + 4 * kg;
     if (f >= F) continue;   // past a ragged last tile (F is a multiple of 4)
-    f16x4 b4 = {};
-    if (bias) b4 = *(const f16x4*)(bias + f);
+    const f16x4 b4 = bias.at(f);
 #pragma unroll
     for (int q = 0; q < TB; ++q) {
       const int tt = t0 + wt * TW + 16 * q + i;
       if (tt >= T) continue;
-      store_out(y + (size_t)tt * ldy + f, acc[xx][q], rs ? rs[tt] : 1.0f, b4, ybf);
+      if (un.P > 1) *(f32x4*)(sp.at(un, kBT * BF) + (tt - t0) * BF + (f - f0)) = acc[xx][q];
+      else store_out(y + (size_t)tt * ldy + f, acc[xx][q], rs ? rs[tt] : 1.0f, b4, ybf);
     }
   }
 }
@@ -1370,6 +1406,35 @@ __global__ __launch_bounds__(256) void k_gemm_split_sum(LinearArgs a, int P, con
   yp[1] = (u32x2){w[2], w[3]};
 }
 
+// The same for the split tiles of the W-streaming GEMM (BF features x 256
+// tokens, placed as there): y = rs[t] · (the parts' sums) + bias in fp16 or
+// (ybf) bf16; 8 features per thread.
+__global__ __launch_bounds__(256) void k_f16w_split_sum(KSplit sp, int BF, int GT, int OB, int F, int T, BiasCols bias,
+                                                        uint16_t* __restrict__ y, int ldy,
+                                                        const float* __restrict__ rs, int ybf) {
+  const int per = 256 * BF / 8;   // threads of a tile: a multiple of the workgroup
+  const int i = (int)(blockIdx.x * 256 + threadIdx.x);
+  const int tail = sp.tiles - sp.T1, tt = i / per, e = i - tt * per;
+  const int tile = sp.T1 + tt;
+  const int TBn = sp.tiles / OB;
+  const int band = tile / (GT * OB), r = tile - band * GT * OB;
+  const int gt = min(GT, TBn - band * GT);
+  const int ob = r / gt, tb = band * GT + r % gt;
+  const int tl = e / (BF / 8), fl = (e - tl * (BF / 8)) * 8;
+  const int t = tb * 256 + tl, f = ob * BF + fl;
+  if (t >= T || f >= F) return;
+  f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = s0;
+  for (int p = 0; p < sp.P; ++p) {
+    const float* q = sp.part + ((size_t)p * tail + tt) * (256 * (size_t)BF) + (size_t)tl * BF + fl;
+    s0 += *(const f32x4*)q;
+    s1 += *(const f32x4*)(q + 4);
+  }
+  const float sc = rs ? rs[t] : 1.0f;
+  uint16_t* yp = y + (size_t)t * ldy + f;
+  store_out(yp, s0, sc, bias.at(f), ybf);
+  store_out(yp + 4, s1, sc, bias.at(f + 4), ybf);
+}
+
 template <bool HAS_S>
 __global__ __launch_bounds__(kGT, 2) void k_gemm_e8d4(LinearArgs a, int OB) {
   gemm_tile<KIND_E8D4, HAS_S>(a, OB);
@@ -1391,69 +1456,91 @@ size_t static_lds(const void* kern) {
 }
 }  // namespace
 
+namespace {
+// Tile width (0: none fits) and K split of the LDS-decode kernel, and the
+// estimated time in us.  Whole 8-, 16-, 20- or 32-Q-row tiles.  Of the two
+// wide tiles, the one with less work per CU (rounds of the CUs x tile width)
+// wins; on a tie the wider tile.
+struct LdsPlan {
+  int bf, P;
+  double us;
+};
+
+LdsPlan plan_lds(int M, int N, int B, size_t room) {
+  const long TB = (B + g3::kBT - 1) / g3::kBT;
+  const long cus = dec::cu_count();
+  long cost160 = -1, cost256 = -1;
+  if (M % 20 == 0) cost160 = ((M / 20) * TB + cus - 1) / cus * 160;
+  if (M % 32 == 0) cost256 = ((M / 32) * TB + cus - 1) / cus * 256;
+  int bf = cost160 < 0 ? (cost256 < 0 ? 0 : 256) : (cost256 < 0 || cost160 < cost256 ? 160 : 256);
+  // 128-feature tiles in place of 256: twice the workgroups, each ~0.8 of
+  // the time (its producers decode in one pass), so they win when
+  // 0.8 x their rounds of the CUs is below the 256 tiles' rounds.
+  if (bf != 160 && M % 16 == 0) {
+    const long r128 = ((M / 16) * TB + cus - 1) / cus, r256 = ((M / 32) * TB + cus - 1) / cus;
+    if (bf == 0 || 4 * r128 < 5 * r256) bf = 128;
+    // 64-feature tiles when they still fit one round of the CUs: a launch
+    // with few token tiles is bound by each workgroup's serial K-steps,
+    // and narrower tiles shorten each step.
+    if (bf == 128 && (long)(M / 8) * TB <= cus) bf = 64;
+  }
+  // With a workspace the tile width and the K split are chosen together:
+  // time ~ rounds of the CUs x K-steps per part x a tile's step time
+  // (measured ~1.09 / 1.33 / 1.66 / 1.66 us for 64 / 128 / 160 / 256
+  // features on 4096-5120-column layers), plus the parts' fp32 sums
+  // written and read once at ~4 TB/s and the summing launch (~3 us).
+  int P = 1;
+  if (bf && room) {
+    const int nk = N / g3::kBK;
+    const double per = (double)B * 8 * M * 4;
+    const int widths[4] = {64, 128, 160, 256};
+    const double step[4] = {1.09, 1.33, 1.66, 1.66};
+    double best = -1;
+    int bw = bf, bp = 1;
+    for (int wi = 0; wi < 4; ++wi) {
+      const int w = widths[wi];
+      if (M % (w / 8) != 0) continue;
+      const long gw = (M / (w / 8)) * TB;
+      for (int pp = 1; pp <= kPrefillMaxParts; ++pp) {
+        if (pp > 1 && (gw * pp > cus || nk / pp < 8 || (size_t)(pp * per) > room)) break;
+        const double t = (double)((gw * pp + cus - 1) / cus) * ((nk + pp - 1) / pp) * step[wi] +
+                         (pp > 1 ? 2.0 * pp * per / 4.0e6 + 3.0 : 0.0);
+        if (best < 0 || t < best) {
+          best = t;
+          bw = w;
+          bp = pp;
+        }
+      }
+    }
+    // An unsplit choice keeps the measured width rule above.
+    if (bp > 1) {
+      bf = bw;
+      P = bp;
+    }
+  }
+  // (The wide tiles' step: 1.5 us in split launches, 1.85 and more, with the
+  // critical blocks, in whole ones.)
+  const double w = bf == 64 ? 1.09 : bf == 128 ? 1.33 : P > 1 ? 1.5 : 1.85;
+  const long g = bf ? (long)(M / (bf / 8)) * TB * P : 0;
+  const int nk = N / g3::kBK;
+  const double us = (double)((g + cus - 1) / cus) * ((nk + P - 1) / P) * w +
+                    (P > 1 ? 2.0 * P * B * 8.0 * M * 4 / 4.0e6 + 3.0 : 0.0);
+  return {bf, P, us};
+}
+}  // namespace
+
 template <int KIND>
 int launch_gemm(const LinearArgs& a, hipStream_t s, void* work, long long work_bytes) {
   if (KIND == KIND_E8D4 && a.B <= kWideMaxTokens && launch_decode_wide_multi(&a, 1, s, work, work_bytes) == 0)
     return 0;
   // LDS-decode kernel: fp16 x and table, no S_group, K-steps of 64, whole
-  // 8-, 16-, 20- or 32-Q-row tiles, 16-byte x rows and 8-byte y stores.  Of the two
-  // tile widths, the one with less work per CU (rounds of the CUs × tile
-  // width) wins; on a tie the wider tile.
+  // 8-, 16-, 20- or 32-Q-row tiles, 16-byte x rows and 8-byte y stores.
   if (KIND == KIND_E8D4 && !a.x_bf16 && !a.codes_f32 && !a.S && a.prep == 0 && (a.N % g3::kBK) == 0 &&
       (a.ldx % 8) == 0 && ((uintptr_t)a.x & 15) == 0 && (a.ldy % 4) == 0 && ((uintptr_t)a.y & 7) == 0) {
     const long TB = (a.B + g3::kBT - 1) / g3::kBT;
-    const long cus = dec::cu_count();
-    long cost160 = -1, cost256 = -1;
-    if (a.M % 20 == 0) cost160 = ((a.M / 20) * TB + cus - 1) / cus * 160;
-    if (a.M % 32 == 0) cost256 = ((a.M / 32) * TB + cus - 1) / cus * 256;
-    int bf = cost160 < 0 ? (cost256 < 0 ? 0 : 256) : (cost256 < 0 || cost160 < cost256 ? 160 : 256);
-    // 128-feature tiles in place of 256: twice the workgroups, each ~0.8 of
-    // the time (its producers decode in one pass), so they win when
-    // 0.8 x their rounds of the CUs is below the 256 tiles' rounds.
-    if (bf != 160 && a.M % 16 == 0) {
-      const long r128 = ((a.M / 16) * TB + cus - 1) / cus, r256 = ((a.M / 32) * TB + cus - 1) / cus;
-      if (bf == 0 || 4 * r128 < 5 * r256) bf = 128;
-      // 64-feature tiles when they still fit one round of the CUs: a launch
-      // with few token tiles is bound by each workgroup's serial K-steps,
-      // and narrower tiles shorten each step.
-      if (bf == 128 && (long)(a.M / 8) * TB <= cus) bf = 64;
-    }
-    // With a workspace the tile width and the K split are chosen together:
-    // time ~ rounds of the CUs x K-steps per part x a tile's step time
-    // (measured ~1.09 / 1.33 / 1.66 / 1.66 us for 64 / 128 / 160 / 256
-    // features on 4096-5120-column layers), plus the parts' fp32 sums
-    // written and read once at ~4 TB/s and the summing launch (~3 us).
-    int P = 1;
     const size_t woff = (size_t)decode_mfma_work_bytes();
-    const size_t wavail = work && work_bytes > (long long)woff ? (size_t)work_bytes - woff : 0;
-    if (bf && wavail) {
-      const int nk = a.N / g3::kBK;
-      const double per = (double)a.B * 8 * a.M * 4;
-      const int widths[4] = {64, 128, 160, 256};
-      const double step[4] = {1.09, 1.33, 1.66, 1.66};
-      double best = -1;
-      int bw = bf, bp = 1;
-      for (int wi = 0; wi < 4; ++wi) {
-        const int w = widths[wi];
-        if (a.M % (w / 8) != 0) continue;
-        const long gw = (a.M / (w / 8)) * TB;
-        for (int pp = 1; pp <= kPrefillMaxParts; ++pp) {
-          if (pp > 1 && (gw * pp > cus || nk / pp < 8 || (size_t)(pp * per) > wavail)) break;
-          const double t = (double)((gw * pp + cus - 1) / cus) * ((nk + pp - 1) / pp) * step[wi] +
-                           (pp > 1 ? 2.0 * pp * per / 4.0e6 + 3.0 : 0.0);
-          if (best < 0 || t < best) {
-            best = t;
-            bw = w;
-            bp = pp;
-          }
-        }
-      }
-      // An unsplit choice keeps the measured width rule above.
-      if (bp > 1) {
-        bf = bw;
-        P = bp;
-      }
-    }
+    const LdsPlan pl = plan_lds(a.M, a.N, a.B, work && work_bytes > (long long)woff ? (size_t)work_bytes - woff : 0);
+    const int bf = pl.bf, P = pl.P;
     const long grid = bf ? (a.M / (bf / 8)) * TB : 0;
     if (bf && grid <= 0x7fffffff) {
       // 160-feature tiles: 8 producer waves (the MFMA waves fit four waves per
@@ -1548,54 +1635,107 @@ int launch_gemm(const LinearArgs& a, hipStream_t s, void* work, long long work_b
   return 0;
 }
 
-// Returns 0 if launched, -1 if the shape is outside k_gemm_f16w: F a
-// multiple of 64, N of 64, x rows 16-byte aligned, y rows 8-byte aligned.
-int launch_gemm_f16w(const uint16_t* W, const uint16_t* x, const f16* bias, int F, int N, int T, int ldx,
-                     uint16_t* y, int ldy, hipStream_t s, const float* rs, int ybf) {
-  if (T <= 0 || F % 64 != 0 || N % g3::kBK != 0 || ldx % 8 != 0 || ((uintptr_t)x & 15) != 0 || ldy % 4 != 0 ||
-      ((uintptr_t)y & 7) != 0 || ((uintptr_t)W & 15) != 0 || (bias && ((uintptr_t)bias & 7) != 0))
-    return -1;
-  // Tile: the one with the least time, rounds of the CUs x one tile's
-  // K-step time (measured 1.08 / 1.64 / 0.88 / 0.65 us at 64 columns for
-  // 160 / 256 / 128 / 64 features x 256 tokens: per unit of area the
-  // narrowest is ~1.5x the others), the earlier one on ties.  The
-  // three-stage kernel takes a ragged last feature tile (F a multiple of
-  // 64, not of the tile), the two-stage 256 x 256 one whole tiles only.  (A
-  // 288 x 128 tile, three whole rounds for 13824 features at 2048 tokens,
-  // measured slower than 256 x 256 with its second round partly idle.)
-  struct Tile { int bf, bt, step; bool ragged; };
-  constexpr Tile tiles[4] = {{160, 256, 108, true}, {256, 256, 164, false}, {128, 256, 88, true}, {64, 256, 65, true}};
+namespace {
+// Tile and K split of a W-streaming GEMM and its estimated time in us: rounds
+// of the CUs x K-steps x one tile's K-step time (measured 1.08 / 1.64 / 0.88 /
+// 0.65 us at 64 columns for 160 / 256 / 128 / 64 features x 256 tokens: per
+// unit of area the narrowest is ~1.5x the others), the earlier tile on ties.
+// Either every tile is split over P workgroups (few tiles), or whole rounds
+// of the CUs run unsplit and only the tiles of the last, partial round are
+// split (22016 features at 512 tokens: 276 tiles of 160 take one round and 20
+// tiles in 8 parts); the split tiles' fp32 sums are written and read once, by
+// a launch of its own (~4 us).  The three-stage kernel takes a ragged last
+// feature tile (F a multiple of 64, not of the tile), the two-stage 256 x 256
+// one whole tiles only.  (A 288 x 128 tile, three whole rounds for 13824
+// features at 2048 tokens, measured slower than 256 x 256 with its second
+// round partly idle.)
+struct F16wPlan {
+  int tile, T1, P;
+  double us;
+};
+struct F16wTile { int bf; double step; bool ragged; };
+constexpr F16wTile kF16wTiles[4] = {{160, 1.08, true}, {256, 1.64, false}, {128, 0.88, true}, {64, 0.65, true}};
+constexpr int kF16wTokens = 256, kF16wMaxParts = 8;
+
+F16wPlan plan_f16w(int F, int N, int T, size_t room) {
   const long cus = dec::cu_count();
-  int k = -1;
-  long best = -1;
+  const int nk = N / g3::kBK;
+  F16wPlan best = {-1, 0, 1, 0.0};
   for (int c = 0; c < 4; ++c) {
-    if (F % tiles[c].bf != 0 && !tiles[c].ragged) continue;
-    const long n = (long)((F + tiles[c].bf - 1) / tiles[c].bf) * ((T + tiles[c].bt - 1) / tiles[c].bt);
-    const long cost = (n + cus - 1) / cus * tiles[c].step;
-    if (k < 0 || cost < best) {
-      best = cost;
-      k = c;
+    const F16wTile& t = kF16wTiles[c];
+    if (F % t.bf != 0 && !t.ragged) continue;
+    const long n = (long)((F + t.bf - 1) / t.bf) * ((T + kF16wTokens - 1) / kF16wTokens);
+    if (n > 0x3fffffff) continue;
+    for (int P = 1; P <= kF16wMaxParts; ++P) {
+      const long T1 = P == 1 ? n : n / cus * cus, tail = n - T1;
+      const double sums = (double)P * tail * t.bf * kF16wTokens * 4;
+      if (P > 1 && (tail == 0 || nk / P < 4 || sums > (double)room)) break;
+      const double us = (P == 1 ? (double)((n + cus - 1) / cus) * nk * t.step
+                                : (double)(n / cus) * nk * t.step +
+                                      (double)((tail * P + cus - 1) / cus) * ((nk + P - 1) / P) * t.step +
+                                      2.0 * sums / 5.0e6 + 4.0);
+      if (best.tile < 0 || us < best.us - 1e-9) best = {c, (int)T1, P, us};
     }
   }
-  const int OB = (F + tiles[k].bf - 1) / tiles[k].bf;
-  const long grid = (long)OB * ((T + tiles[k].bt - 1) / tiles[k].bt);
+  return best;
+}
+}  // namespace
+
+double f16w_estimate_us(int F, int N, int T, size_t room) { return plan_f16w(F, N, T, room).us; }
+
+double fused_estimate_us(int M, int N, int T, size_t room) {
+  const LdsPlan pl = plan_lds(M, N, T, room);
+  return pl.bf && N % g3::kBK == 0 ? pl.us : -1.0;
+}
+
+// Returns 0 if launched, -1 if the shape is outside k_gemm_f16w: F a
+// multiple of 64, N of 64, x rows 16-byte aligned, y rows 8-byte aligned.
+// Layer l's features start at starts[l] (ascending from 0); work: see
+// kernels.h.
+int launch_gemm_f16w(const uint16_t* W, const uint16_t* x, int n_layers, const f16* const* biases, const int* starts,
+                     int F, int N, int T, int ldx, uint16_t* y, int ldy, hipStream_t s, const float* rs, int ybf,
+                     void* work, long long work_bytes) {
+  if (T <= 0 || F % 64 != 0 || N % g3::kBK != 0 || ldx % 8 != 0 || ((uintptr_t)x & 15) != 0 || ldy % 4 != 0 ||
+      ((uintptr_t)y & 7) != 0 || ((uintptr_t)W & 15) != 0 || n_layers < 1 || n_layers > kMaxLayers)
+    return -1;
+  BiasCols bias;
+  for (int l = 0; l < kMaxLayers; ++l) {
+    bias.b[l] = l < n_layers ? biases[l] : nullptr;
+    bias.start[l] = l < n_layers ? starts[l] : 0x7fffffff;
+    if (((uintptr_t)bias.b[l] & 7) != 0) return -1;
+  }
+  const size_t off = (size_t)decode_mfma_work_bytes();
+  const size_t room = work && work_bytes > (long long)off ? (size_t)work_bytes - off : 0;
+  const F16wPlan pl = plan_f16w(F, N, T, room);
+  const int k = pl.tile;
+  if (k < 0) return -1;
+  const int OB = (F + kF16wTiles[k].bf - 1) / kF16wTiles[k].bf;
+  const int tiles = OB * ((T + kF16wTokens - 1) / kF16wTokens);
+  const KSplit sp = {tiles, pl.T1, pl.P, pl.P > 1 ? (float*)((char*)work + off) : nullptr};
+  const long grid = pl.T1 + (long)(tiles - pl.T1) * pl.P;
   if (grid > 0x7fffffff) return -1;
   auto run = [&](auto kern, int threads, int bytes, int v) {
     static bool attr[4] = {false, false, false, false};
     if (!attr[v]) attr[v] = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) == hipSuccess;
     if (!attr[v]) return -1;
-    kern<<<(unsigned)grid, threads, bytes, s>>>(W, x, bias, N, T, ldx, y, ldy, OB, F, rs, ybf);
+    kern<<<(unsigned)grid, threads, bytes, s>>>(W, x, bias, N, T, ldx, y, ldy, OB, F, rs, ybf, sp);
     return 0;
   };
   // Three stages where they fit the CU's 160 KB of LDS (all but 256 x 256).
   // The 256 x 256 tile runs the two-stage kernel with 8-token-tile bands
   // (measured 4% faster than 4 at 13824 features).
+  int rc;
   switch (k) {
-    case 0: return run(k_gemm_f16w4<160, 256>, 512, 3 * (256 + 160) * 128, 0);
-    case 1: return run(k_gemm_f16w<256, 4, 2, 8>, 768, 2 * (256 + 256) * 128, 1);
-    case 2: return run(k_gemm_f16w4<128, 256>, 512, 3 * (256 + 128) * 128, 2);
-    default: return run(k_gemm_f16w4<64, 256>, 512, 3 * (256 + 64) * 128, 3);
+    case 0: rc = run(k_gemm_f16w4<160, 256>, 512, 3 * (256 + 160) * 128, 0); break;
+    case 1: rc = run(k_gemm_f16w<256, 4, 2, 8>, 768, 2 * (256 + 256) * 128, 1); break;
+    case 2: rc = run(k_gemm_f16w4<128, 256>, 512, 3 * (256 + 128) * 128, 2); break;
+    default: rc = run(k_gemm_f16w4<64, 256>, 512, 3 * (256 + 64) * 128, 3); break;
   }
+  if (rc == 0 && pl.P > 1) {
+    const int bf = kF16wTiles[k].bf, gt = k == 1 ? 8 : 4;
+    k_f16w_split_sum<<<(unsigned)((tiles - pl.T1) * (bf / 8)), 256, 0, s>>>(sp, bf, gt, OB, F, T, bias, y, ldy, rs, ybf);
+  }
+  return rc;
 }
 
 // bf16 activations for the W-streaming GEMM: row t of x becomes

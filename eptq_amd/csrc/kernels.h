@@ -13,7 +13,7 @@ enum { KIND_E8D4 = 0, KIND_E8 = 1 };
 
 struct DequantArgs {
   const int16_t* Q;
-  const float* table;
+  const void* table;   // fp32, or fp16 (table_f16: each value widened)
   const f16* g;
   const f16* h;
   const f16* O;
@@ -23,6 +23,8 @@ struct DequantArgs {
   int qb;
   int M, N;
   f16* W;
+  int table_f16;
+  int keep;       // W is read next: stores stay in the caches
 };
 
 struct LinearArgs {
@@ -125,10 +127,19 @@ constexpr size_t kSplitCounterBytes = (size_t)kSplitCounters * 4;
 constexpr size_t kSplitPartBytes = (16 * 64 + 16) * 4;
 constexpr int kSplitTileRows = 64;
 // Prefill GEMM over dequantized fp16 weights: y (T, F) = rs[t] · (x (T, N) ·
-// Wᵀ) + bias for W (F, N) row-major, rs NULL for 1, y fp16 or (ybf) bf16;
-// -1 when the shape is outside the kernel.
-int launch_gemm_f16w(const uint16_t* W, const uint16_t* x, const f16* bias, int F, int N, int T, int ldx,
-                     uint16_t* y, int ldy, hipStream_t s, const float* rs = nullptr, int ybf = 0);
+// Wᵀ) + bias for W (F, N) row-major, the biases of n_layers layers side by
+// side (each nullable, first features in starts), rs NULL for 1, y fp16 or
+// (ybf) bf16; -1 when the shape is outside the kernel.  work (nullable): a
+// decode workspace, whose prefill area takes the fp32 sums where tiles that
+// leave CUs idle split K.
+int launch_gemm_f16w(const uint16_t* W, const uint16_t* x, int n_layers, const f16* const* biases, const int* starts,
+                     int F, int N, int T, int ldx, uint16_t* y, int ldy, hipStream_t s, const float* rs = nullptr,
+                     int ybf = 0, void* work = nullptr, long long work_bytes = 0);
+// Its estimated time (room: bytes for split sums).
+double f16w_estimate_us(int F, int N, int T, size_t room);
+// The fused fp16 prefill kernel's (one E8-D4 layer without S_group), negative
+// where it does not take the shape.
+double fused_estimate_us(int M, int N, int T, size_t room);
 // bf16 rows to fp16 for it: x16[t] = fp16(x[t] · 2^-e_t), rs[t] = 2^e_t.
 int launch_bf16_rows_to_f16(const uint16_t* x, int N, int T, uint16_t* x16, float* rs, hipStream_t s);
 // Workspace bytes that let the matrix-core decode split every launch it takes.

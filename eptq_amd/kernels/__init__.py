@@ -79,9 +79,8 @@ def _check_layer(kind, Q, codes, g, h, O_vals, O_col, O_row_ptr, S_group):
 def linear_forward(kind: str, Q, codes, g, h, x, O_vals, O_col, O_row_ptr, bias=None,
                    S_group=None, two_pass: bool = False) -> torch.Tensor:
     """Run the fused quantized Linear on ``x`` (B, N) -> (B, 8M), dtype of x.
-    ``two_pass`` (what the module's ops pass): from ``_two_pass_min`` tokens
-    (2048 for E8-D4, 256 with S_group or bf16 x, 64 for E8) and 64-multiple
-    shapes, the two-pass prefill instead of the fused C-ABI kernel."""
+    ``two_pass`` (what the module's ops pass): the two-pass prefill instead of
+    the fused C-ABI kernel where it is preferred (``_two_pass_into``)."""
     M, N, n_groups = _check_layer(kind, Q, codes, g, h, O_vals, O_col, O_row_ptr, S_group)
     _require(x.device == Q.device, "x must be on the layer's device")
     _require(x.dim() == 2 and x.shape[1] == N, f"x must be (B, {N})")
@@ -95,10 +94,11 @@ def linear_forward(kind: str, Q, codes, g, h, x, O_vals, O_col, O_row_ptr, bias=
     if B == 0:
         return y
     lib = _lib.load()
-    layer = dict(Q=Q, g=g, h=h, O_vals=O_vals, O_col=O_col, O_row_ptr=O_row_ptr, bias=bias, S_group=S_group)
-    if two_pass and B >= _two_pass_min(kind, [layer], x) and _two_pass_ok([layer], x, N):
-        _two_pass_into(lib, [layer], codes, x, y, kind)
-        return y
+    if two_pass and B >= (TWO_PASS_MIN_TOKENS if kind == "e8_d4" else TWO_PASS_MIN_TOKENS_E8):
+        layer = dict(Q=Q, g=g, h=h, O_vals=O_vals, O_col=O_col, O_row_ptr=O_row_ptr, bias=bias, S_group=S_group)
+        arr = (_lib.EptqLayer * 1)(_layer_entry(layer, M, n_groups, 0))
+        if _two_pass_into(lib, arr, codes, x, y, kind, stream_workspace(x.device)):
+            return y
     fn = lib.eptq_e8d4_forward if kind == "e8_d4" else lib.eptq_e8_forward
     with torch.cuda.device(x.device):
         stream = torch.cuda.current_stream().cuda_stream
@@ -175,72 +175,46 @@ def _workspace_outside_graph_pools(device, stream) -> torch.Tensor:
     return box["w"]
 
 
-# Token counts from which the module's forwards run the two-pass prefill
-# (every weight decoded once into a transient fp16 W, then eptq_f16_gemm).
-# E8-D4: measured 1.09-1.36x the fused kernel at 2048 tokens on the six
-# Llama-2-7B / 13B projection shapes, mixed at 1024 (0.85-1.11x: the fused
-# kernel splits K over idle CUs there), slower at 512.  E8-D4 with S_group
-# (whose fused path is the older grouped GEMM): 1.2-1.8x from 256 tokens on
-# 4096x4096, 11008x4096 and 4096x11008.  E8 (whose fused GEMM gathers from a
-# 1 MB table): 2x from 64 tokens on 4096x4096, 1.3-2.5x at 256-2048 tokens on
-# 4096x4096 and 11008x4096, level on 3072x768.  E8-D4 with bf16 x (whose
-# fused path decodes into registers): 1.2-2.1x from 256 tokens on 4096x4096,
-# 11008x4096, 4096x11008 and 14336x4096.
-TWO_PASS_MIN_TOKENS = 2048
-TWO_PASS_MIN_TOKENS_GROUPED = 256
-TWO_PASS_MIN_TOKENS_BF16 = 256
-TWO_PASS_MIN_TOKENS_E8 = 64
+# The least token counts at which the module's forwards may run the two-pass
+# prefill (every weight decoded once into a transient fp16 W, then the
+# W-streaming GEMM); ``eptq_two_pass_scratch_bytes`` decides.  E8 layers, whose
+# fused GEMM gathers from a 1 MB table: 2.1x at 17 rows on 4096x4096, 1.5x on
+# 11008x4096, 2.6x on 4096x11008.  E8-D4 with S_group or bf16 x: a Llama-2-7B
+# layer at 130 rows 984 -> 278 us (bf16), 3022 -> 279 us (bf16 with S_group).
+# E8-D4 otherwise: by estimated times, between 129 and 2048 rows either may win.
+TWO_PASS_MIN_TOKENS_E8 = 17
+TWO_PASS_MIN_TOKENS = 129
 
 
-def _two_pass_min(kind: str, layers, x) -> int:
-    if kind != "e8_d4":
-        return TWO_PASS_MIN_TOKENS_E8
-    if x.dtype == torch.bfloat16:
-        return TWO_PASS_MIN_TOKENS_BF16
-    return TWO_PASS_MIN_TOKENS_GROUPED if all(L.get("S_group") is not None for L in layers) else TWO_PASS_MIN_TOKENS
-
-
-def _two_pass_ok(layers, x, N) -> bool:
-    # bf16 x goes through eptq_bf16_rows_to_f16 (rows up to 16384 columns).
-    return ((x.dtype == torch.float16 or (x.dtype == torch.bfloat16 and N <= 16384)) and N % 64 == 0
-            and all((8 * int(L["Q"].shape[0])) % 64 == 0 for L in layers))
-
-
-def _two_pass_into(lib, layers, codes, x, y, kind: str = "e8_d4") -> None:
+def _two_pass_into(lib, arr, codes, x, y, kind: str, work: Optional[torch.Tensor], always: bool = False) -> bool:
     """y[:, layer columns] = x · W_lᵀ + bias_l with each layer's W decoded once
-    (``eptq_e8d4_dequant`` / ``eptq_e8_dequant``, S_group included, into one
-    transient buffer sized for the largest layer, reused layer after layer on
-    the stream) and multiplied by ``eptq_f16_gemm_rows``.  The table is the
-    kernels' (fp16, widened to fp32): the same table values the fused kernel
-    multiplies.  bf16 x is first taken to fp16 row by row with a power-of-two
-    scale (``eptq_bf16_rows_to_f16``) that the GEMM restores at its bf16
-    output."""
-    N = int(x.shape[1])
-    B, ldy = int(x.shape[0]), int(y.shape[1])
-    tab = codes if codes.dtype == torch.float32 else codes.float()
-    F_max = max(8 * int(L["Q"].shape[0]) for L in layers)
-    wbuf = torch.empty(F_max * N, dtype=torch.float16, device=x.device)
-    deq = lib.eptq_e8d4_dequant if kind == "e8_d4" else lib.eptq_e8_dequant
-    off = 0
+    (S_group included) into a transient buffer and multiplied by the W-streaming
+    GEMM (``eptq_two_pass_forward``; ``arr``: the layers as an ``EptqLayer``
+    array), where that is preferred or ``always`` is set; False where not.  The
+    table is the kernels' (fp16): the same table values the fused kernel
+    multiplies."""
+    B, N, n = x.shape[0], x.shape[1], len(arr)
+    if B < (TWO_PASS_MIN_TOKENS if kind == "e8_d4" else TWO_PASS_MIN_TOKENS_E8) and not always:
+        return False
+    e8, xdt = int(kind != "e8_d4"), EPTQ_BF16 if x.dtype == torch.bfloat16 else EPTQ_F16
     with torch.cuda.device(x.device):
-        stream = torch.cuda.current_stream().cuda_stream
-        xg, rs = x, None
-        if x.dtype == torch.bfloat16:
-            xg = torch.empty((B, N), dtype=torch.float16, device=x.device)
-            rs = torch.empty(B, dtype=torch.float32, device=x.device)
-            _lib.check(lib.eptq_bf16_rows_to_f16(_ptr(x), N, B, _ptr(xg), _ptr(rs), stream), "eptq_bf16_rows_to_f16")
-        y_dtype = EPTQ_BF16 if y.dtype == torch.bfloat16 else EPTQ_F16
-        for L in layers:
-            M = int(L["Q"].shape[0])
-            S = L.get("S_group")
-            n_groups = 0 if S is None else int(S.shape[0])
-            rc = deq(_ptr(L["Q"]), _ptr(tab), _ptr(L["g"]), _ptr(L["h"]), _ptr(L["O_vals"]), _ptr(L["O_col"]),
-                     _ptr(L["O_row_ptr"]), _ptr(S), n_groups, M, N, _ptr(wbuf), stream)
-            _lib.check(rc, deq.__name__)
-            rc = lib.eptq_f16_gemm_rows(_ptr(wbuf), _ptr(xg), _ptr(L.get("bias")), 8 * M, N, B, _ptr(rs),
-                                        _ptr(y) + 2 * off, y_dtype, ldy, stream)
-            _lib.check(rc, "eptq_f16_gemm_rows")
-            off += 8 * M
+        nbytes = lib.eptq_two_pass_scratch_bytes(e8, n, arr, N, B, xdt, int(work is not None), int(always))
+        if nbytes == 0:
+            return False
+        if codes.data_ptr() % 16:
+            codes = codes.clone()
+        scratch = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
+        rc = lib.eptq_two_pass_forward(
+            e8, n, arr, codes.data_ptr(), EPTQ_F32 if codes.dtype == torch.float32 else EPTQ_F16, x.data_ptr(), xdt, N,
+            B, y.data_ptr(), y.shape[1], scratch.data_ptr(), nbytes, _ptr(work), 0 if work is None else work.numel(),
+            torch.cuda.current_stream().cuda_stream)
+    _lib.check(rc, "eptq_two_pass_forward")
+    return True
+
+
+def _layer_entry(L, M: int, n_groups: int, off: int):
+    return _lib.EptqLayer(_ptr(L["Q"]), _ptr(L["g"]), _ptr(L["h"]), _ptr(L["O_vals"]), _ptr(L["O_col"]),
+                          _ptr(L["O_row_ptr"]), _ptr(L.get("bias")), _ptr(L.get("S_group")), n_groups, M, off)
 
 
 def linear_forward_multi(layers, codes, x, work: Optional[torch.Tensor] = None,
@@ -249,9 +223,8 @@ def linear_forward_multi(layers, codes, x, work: Optional[torch.Tensor] = None,
     side by side, in one decode launch when the kernel takes them all.
     ``layers``: dicts with Q, g, h, O_vals, O_col, O_row_ptr and optional
     bias, S_group (the EPTQLinear buffers).  ``two_pass`` (what the
-    module's op passes): from ``_two_pass_min`` fp16 tokens (64-multiple
-    shapes) the two-pass prefill (``_two_pass_into``) instead of the fused
-    C-ABI launch.  ``work``: optional workspace from
+    module's op passes): the two-pass prefill (``_two_pass_into``) instead of
+    the fused C-ABI launch where it is preferred.  ``work``: optional workspace from
     ``decode_workspace`` (lets batches of 3..16 split the columns of layers
     with few row tiles over several workgroups); calls sharing one must not
     overlap in time."""
@@ -261,23 +234,18 @@ def linear_forward_multi(layers, codes, x, work: Optional[torch.Tensor] = None,
     N = int(x.shape[1])
     arr = (_lib.EptqLayer * len(layers))()
     off = 0
-    keep = []
     for i, L in enumerate(layers):
         M, n2, n_groups = _check_layer("e8_d4", L["Q"], codes, L["g"], L["h"], L["O_vals"], L["O_col"],
                                        L["O_row_ptr"], L.get("S_group"))
         _require(n2 == N and L["Q"].device == x.device, "layers must take x's in_features on x's device")
-        b = L.get("bias")
-        arr[i] = _lib.EptqLayer(_ptr(L["Q"]), _ptr(L["g"]), _ptr(L["h"]), _ptr(L["O_vals"]), _ptr(L["O_col"]),
-                                _ptr(L["O_row_ptr"]), _ptr(b), _ptr(L.get("S_group")), n_groups, M, off)
+        arr[i] = _layer_entry(L, M, n_groups, off)
         off += 8 * M
-        keep.append(L)
     B = int(x.shape[0])
     y = torch.empty((B, off), dtype=x.dtype, device=x.device)
     if B == 0:
         return y
     lib = _lib.load()
-    if two_pass and B >= _two_pass_min("e8_d4", keep, x) and _two_pass_ok(keep, x, N):
-        _two_pass_into(lib, keep, codes, x, y)
+    if two_pass and _two_pass_into(lib, arr, codes, x, y, "e8_d4", work):
         return y
     with torch.cuda.device(x.device):
         stream = torch.cuda.current_stream().cuda_stream

@@ -31,6 +31,9 @@ SIGNATURES = {
     "eptq_f16_gemm": ([_P, _P, _P, _I, _I, _I, _P, _I, _P], _I),
     "eptq_f16_gemm_rows": ([_P, _P, _P, _I, _I, _I, _P, _P, _I, _I, _P], _I),
     "eptq_bf16_rows_to_f16": ([_P, _I, _I, _P, _P, _P], _I),
+    "eptq_two_pass_forward": ([_I, _I, _P, _P, _I, _P, _I, _I, _I, _P, _I, _P, ctypes.c_longlong, _P,
+                               ctypes.c_longlong, _P], _I),
+    "eptq_two_pass_scratch_bytes": ([_I, _I, _P, _I, _I, _I, _I, _I], ctypes.c_longlong),
 }
 
 class EptqLayer(ctypes.Structure):

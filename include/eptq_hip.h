@@ -195,6 +195,34 @@ int eptq_f16_gemm_rows(const void* W, const void* x, const void* bias, int F, in
  */
 int eptq_bf16_rows_to_f16(const void* x, int N, int T, void* x16, void* row_scale, void* stream);
 
+/*
+ * Two-pass prefill of n_layers layers that share x: each layer's W from the
+ * dequantizer into scratch, then the W-streaming GEMM, y[:, layer columns] =
+ * x · W_lᵀ + bias_l in x's type (bf16 x by way of eptq_bf16_rows_to_f16).
+ * Where one GEMM over all layers is estimated faster (layers with few rows
+ * leave CUs idle alone) scratch holds all their W, otherwise one layer's at a
+ * time.  e8: 0 E8-D4, 1 E8 layers; codes: the table, fp32 or fp16
+ * (codes_dtype; fp16 values are widened); scratch: 256-byte aligned, of
+ * eptq_two_pass_scratch_bytes() bytes (fewer, down to one layer's W, run the
+ * layers one at a time); work: NULL or a workspace as in
+ * eptq_e8d4_forward_multi, whose prefill area takes split-K sums.  M of every
+ * layer a multiple of 8, N of 64 (and up to 16384 for bf16 x); x, y and
+ * scratch must not overlap.  No counterpart in the reference (as
+ * eptq_f16_gemm).
+ */
+int eptq_two_pass_forward(int e8, int n_layers, const eptq_layer* layers, const void* codes, int codes_dtype,
+                          const void* x, int x_dtype, int N, int B, void* y, int ldy, void* scratch,
+                          long long scratch_bytes, void* work, long long work_bytes, void* stream);
+
+/*
+ * Scratch bytes of that call, or 0 where it cannot take the shape or (always
+ * = 0) the fused launches are estimated faster.  Preferred are E8 layers from
+ * 17 rows, E8-D4 with S_group or bf16 x from 129 (their fused kernels are 2 to
+ * 20 times slower), and E8-D4 otherwise from 129 by the estimated times.
+ */
+long long eptq_two_pass_scratch_bytes(int e8, int n_layers, const eptq_layer* layers, int N, int B, int x_dtype,
+                                      int has_work, int always);
+
 int eptq_e8_dequant(const void* Q, const void* codes_f32,
                     const void* g, const void* h,
                     const void* O_vals, const void* O_col, const void* O_row_ptr,

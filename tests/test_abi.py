@@ -233,3 +233,55 @@ def test_noalloc_checks_like_the_workspace_form(lib):
         assert rc_w == rc_n == want, (n, N, B, ldy, rc_w, rc_n)
         if want:
             assert msg_n.replace("_noalloc", "") == msg_w, (msg_w, msg_n)
+
+
+def _two_pass_layers(*Ms, **over):
+    arr = (_lib.EptqLayer * len(Ms))()
+    off = 0
+    for k, M in enumerate(Ms):
+        arr[k] = _lib.EptqLayer(16, 16, 16, None, None, 16, over.get("bias"), None, 0, M, off)
+        off += 8 * M
+    return arr, off
+
+
+@pytest.mark.parametrize("over,code,msg", [
+    (dict(x=None), _lib.EPTQ_EINVAL, "null"),
+    (dict(codes_dtype=7), _lib.EPTQ_EINVAL, "codes_dtype"),
+    (dict(x_dtype=_lib.EPTQ_F32), _lib.EPTQ_EINVAL, "x_dtype"),
+    (dict(N=96), _lib.EPTQ_EUNSUPPORTED, "multiple of 64"),
+    (dict(N=16448, x_dtype=_lib.EPTQ_BF16), _lib.EPTQ_EUNSUPPORTED, "16384"),
+    (dict(M=12), _lib.EPTQ_EUNSUPPORTED, "multiple of 8"),
+    (dict(scratch_bytes=100), _lib.EPTQ_EINVAL, "scratch of"),
+    (dict(scratch=(1 << 20) + 16), _lib.EPTQ_EUNSUPPORTED, "alignment"),
+    (dict(scratch=1 << 20), _lib.EPTQ_EINVAL, "overlap"),
+    (dict(ldy=64), _lib.EPTQ_EINVAL, "outside"),
+    (dict(work=8), _lib.EPTQ_EINVAL, "work"),
+])
+def test_two_pass_forward_rejects_invalid_arguments(lib, over, code, msg):
+    a = dict(e8=0, n=2, M=16, codes=16, codes_dtype=_lib.EPTQ_F16, x=1 << 20, x_dtype=_lib.EPTQ_F16, N=64, B=40,
+             y=1 << 24, ldy=256, scratch=1 << 28, scratch_bytes=1 << 20, work=None, work_bytes=0)
+    a.update(over)
+    arr, _ = _two_pass_layers(a["M"], 16)
+    rc = lib.eptq_two_pass_forward(a["e8"], a["n"], arr, a["codes"], a["codes_dtype"], a["x"], a["x_dtype"], a["N"],
+                                   a["B"], a["y"], a["ldy"], a["scratch"], a["scratch_bytes"], a["work"],
+                                   a["work_bytes"], None)
+    assert rc == code, lib.eptq_last_error()
+    assert msg in lib.eptq_last_error().decode()
+
+
+def test_two_pass_scratch_and_preference(lib):
+    """One layer's W or all of them; E8 from 17 rows, E8-D4 with bf16 x from 129, fp16 E8-D4 by estimated time."""
+    f16, bf16 = _lib.EPTQ_F16, _lib.EPTQ_BF16
+    need = lib.eptq_two_pass_scratch_bytes
+    one, _ = _two_pass_layers(512)
+    W = 2 * 4096 * 4096
+    assert need(0, 1, one, 4096, 2048, f16, 1, 1) == W
+    assert need(0, 1, one, 4096, 2048, bf16, 1, 1) == W + 2 * 2048 * 4096 + 4 * 2048
+    gqa, _ = _two_pass_layers(512, 128, 128)     # q, k, v: k and v alone would leave most CUs idle
+    assert need(0, 3, gqa, 4096, 1000, f16, 1, 0) == 2 * 6144 * 4096
+    many, _ = _two_pass_layers(*[512] * 6)        # more than one launch takes
+    assert need(0, 6, many, 4096, 1000, f16, 1, 1) == W
+    assert need(1, 1, one, 4096, 17, f16, 1, 0) == W and need(1, 1, one, 4096, 16, f16, 1, 0) == 0
+    assert need(0, 1, one, 4096, 128, bf16, 1, 0) == 0 and need(0, 1, one, 4096, 129, bf16, 1, 0) > W
+    assert need(0, 1, one, 16448, 129, bf16, 1, 1) == 0 and need(0, 1, one, 4104, 129, f16, 1, 1) == 0
+    assert need(0, 1, one, 4096, 2048, f16, 1, 0) == W and need(0, 1, one, 4096, 129, f16, 1, 0) == 0

@@ -16,6 +16,7 @@ import pytest
 import torch
 
 from eptq_amd.kernels import _lib, dequant, f16_gemm
+from eptq_amd.kernels.linear import EPTQLinear
 from eptq_amd.quantizers import E8D4Quantizer
 from eptq_amd.synthetic import make_layer, make_x
 from oracle.matvec import linear_ref, rel_l2
@@ -121,3 +122,38 @@ def test_f16_gemm_unsupported():
     with pytest.raises(_lib.EptqError) as err:
         f16_gemm(W, x)
     assert err.value.code == _lib.EPTQ_EUNSUPPORTED
+
+
+# Two-pass calls that split K: every tile (few tiles), the tail of a partial last round (a ragged 160-wide tile on
+# 22016 features), token counts off the 256-token tile; q|k|v of unequal heights in one GEMM with a bias on one.
+# Bound: W and y round by at most 2^-11 of their value each, bf16 outputs by 2^-9.
+@pytest.mark.parametrize("outs,inp,T,dt,qb", [
+    ((64,), 512, 130, torch.float16, None),
+    ((1024,), 4096, 257, torch.bfloat16, None),
+    ((22016,), 768, 500, torch.float16, None),
+    ((4096, 1024, 1024), 1024, 300, torch.float16, 128),
+    ((1088, 64, 192), 2048, 1000, torch.bfloat16, 64),
+])
+def test_two_pass_split_and_together(outs, inp, T, dt, qb):
+    from eptq_amd.kernels import _layer_entry, _lib, _two_pass_into, decode_workspace
+    print(f"two-pass {outs}x{inp} T={T} {dt}", flush=True)
+    tab = table("e8_d4", 1.75)
+    qds = [make_layer(o, inp, seed=o + k, percmask=0.002, bias=(k == 0), qb_size=qb) for k, o in enumerate(outs)]
+    lins = [EPTQLinear.from_quantized_data(qd, torch.from_numpy(tab), "e8_d4").to("cuda:0") for qd in qds]
+    x = make_x(T, inp, seed=T).to(dt).cuda()
+    arr = (_lib.EptqLayer * len(lins))()
+    off = 0
+    for k, l in enumerate(lins):
+        L = {n: getattr(l, n) for n in ("Q", "g", "h", "O_vals", "O_col", "O_row_ptr", "bias", "S_group")}
+        arr[k] = _layer_entry(L, outs[k] // 8, 0 if qb is None else outs[k] // qb, off)
+        off += outs[k]
+    want = torch.cat([x.float() @ l.dequantize().float().t() + (l.bias.float() if l.bias is not None else 0)
+                      for l in lins], dim=-1)
+    got = []
+    for work in (decode_workspace("cuda:0"), None):
+        y = torch.full((T, off), float("nan"), dtype=dt, device="cuda:0")
+        assert _two_pass_into(_lib.load(), arr, lins[0]._codebook, x, y, "e8_d4", work, always=True)
+        got.append(y)
+        err = float((y.float() - want).norm() / want.norm())
+        assert err <= (2.0 ** -8 if dt == torch.bfloat16 else 2.0 ** -10), err
+    assert float((got[0].float() - got[1].float()).norm() / want.norm()) <= (2.0 ** -8 if dt == torch.bfloat16 else 2.0 ** -11)
