@@ -546,7 +546,8 @@ static bool two_pass_shape(int n_layers, const eptq_layer* layers, int N, int B,
   if (n_layers < 1 || !layers || N <= 0 || N % 64 != 0 || B < 1) return false;
   if (x_dtype != EPTQ_F16 && (x_dtype != EPTQ_BF16 || N > 16384)) return false;   // bf16 rows to fp16
   for (int l = 0; l < n_layers; ++l)
-    if (layers[l].M <= 0 || layers[l].M % 8 != 0 || layers[l].M > 0x7fffffff / 64) return false;
+    if (layers[l].M <= 0 || layers[l].M % 8 != 0 || layers[l].M > 0x7fffffff / 64 || ((uintptr_t)layers[l].bias & 7) != 0)
+      return false;   // (bias is read in 8-byte pieces)
   return true;
 }
 
@@ -611,14 +612,13 @@ int eptq_two_pass_forward(int e8, int n_layers, const eptq_layer* layers, const 
   if (work && (!aligned16(work) || work_bytes < 0))
     return fail(EPTQ_EINVAL, "%s: work must be 16-byte aligned with work_bytes >= 0", fn);
   if (!two_pass_shape(n_layers, layers, N, B, x_dtype))
-    return fail(EPTQ_EUNSUPPORTED, "%s: N=%d (a multiple of 64; up to 16384 for bf16 x), M of every layer a multiple of 8", fn, N);
+    return fail(EPTQ_EUNSUPPORTED, "%s: N=%d (a multiple of 64; up to 16384 for bf16 x), M of every layer a multiple of 8, bias 8-byte aligned", fn, N);
   if (!aligned16(x) || ((uintptr_t)scratch & 255) != 0 || ldy % 4 != 0 || ((uintptr_t)y & 7) != 0)
     return fail(EPTQ_EUNSUPPORTED, "%s: ldy=%d (a multiple of 4) or alignment", fn, ldy);
   long long at = 0, sum, most;
   bool packed = true;   // outputs side by side from column 0
   for (int l = 0; l < n_layers; ++l) {
     const eptq_layer& L = layers[l];
-    if (((uintptr_t)L.bias & 7) != 0) return fail(EPTQ_EUNSUPPORTED, "%s: layer %d: bias alignment", fn, l);
     if (L.y_offset < 0 || L.y_offset + 8LL * L.M > (long long)ldy || (L.y_offset & 3))
       return fail(EPTQ_EINVAL, "%s: layer %d columns [%lld, %lld) outside a y row of %d (offset %% 4 == 0)", fn, l,
                   L.y_offset, L.y_offset + 8LL * L.M, ldy);

@@ -22,6 +22,7 @@ sees each quantized Linear as one op with no graph break.
 from __future__ import annotations
 
 
+import contextlib
 import threading
 from typing import List, Optional
 
@@ -46,33 +47,68 @@ def _require(cond: bool, msg: str) -> None:
         raise RuntimeError(msg)
 
 
+def _raw_stream(device: torch.device) -> int:
+    """The current stream of ``device`` as a raw hipStream_t (what
+    ``torch.cuda.current_stream(device).cuda_stream`` is, without the Stream
+    object: 0.3 against 2.8 us)."""
+    return torch._C._cuda_getCurrentRawStream(device.index)
+
+
+_NO_SWITCH = contextlib.nullcontext()
+
+
+def _on(device: torch.device):
+    """A context with ``device`` current (the library launches on the current
+    device); entered without a switch where it already is."""
+    return _NO_SWITCH if device.index == torch.cuda.current_device() else torch.cuda.device(device)
+
+
+def _bad_operand(name: str, t, dev, dt) -> None:
+    _require(t.device == dev, f"{name} must be on {dev}")
+    _require(t.dtype == dt, f"{name} must be {dt}, got {t.dtype}")
+    _require(t.is_contiguous(), f"{name} must be contiguous")
+
+
 def _check_layer(kind, Q, codes, g, h, O_vals, O_col, O_row_ptr, S_group):
-    _require(Q.is_cuda, "Q must be a CUDA (HIP) tensor")
+    # Run on every call: messages are formed only on failure.
+    if not Q.is_cuda:
+        raise RuntimeError("Q must be a CUDA (HIP) tensor")
     dev = Q.device
-    _require(Q.dtype == torch.int16 and Q.dim() == 2 and Q.is_contiguous(),
-             "Q must be a contiguous 2-D int16 tensor")
+    if Q.dtype != torch.int16 or Q.dim() != 2 or not Q.is_contiguous():
+        raise RuntimeError("Q must be a contiguous 2-D int16 tensor")
     M, N = Q.shape
-    for name, t, dt in (("g", g, torch.float16), ("h", h, torch.float16),
-                        ("O_vals", O_vals, torch.float16), ("O_col", O_col, torch.int32),
-                        ("O_row_ptr", O_row_ptr, torch.int32)):
-        _require(t.device == dev, f"{name} must be on {dev}")
-        _require(t.dtype == dt, f"{name} must be {dt}, got {t.dtype}")
-        _require(t.is_contiguous(), f"{name} must be contiguous")
-    _require(g.numel() == 8 * M, f"g must have {8 * M} elements")
-    _require(h.numel() == N, f"h must have {N} elements")
-    _require(O_row_ptr.numel() == M + 1, f"O_row_ptr must have {M + 1} elements")
-    _require(O_vals.numel() == 8 * O_col.numel(), "O_vals must be (nnz, 8) with nnz = len(O_col)")
-    _require(codes.device == dev and codes.is_contiguous(), "codebook must be contiguous on the layer's device")
-    _require(codes.dtype in (torch.float16, torch.float32), "codebook must be fp16 or fp32")
-    rows = 512 if kind == "e8_d4" else 65535
-    _require(codes.numel() == rows * (4 if kind == "e8_d4" else 8),
-             f"{kind} codebook must have {rows} rows")
+    f16, i32 = torch.float16, torch.int32
+    if g.device != dev or g.dtype != f16 or not g.is_contiguous():
+        _bad_operand("g", g, dev, f16)
+    if h.device != dev or h.dtype != f16 or not h.is_contiguous():
+        _bad_operand("h", h, dev, f16)
+    if O_vals.device != dev or O_vals.dtype != f16 or not O_vals.is_contiguous():
+        _bad_operand("O_vals", O_vals, dev, f16)
+    if O_col.device != dev or O_col.dtype != i32 or not O_col.is_contiguous():
+        _bad_operand("O_col", O_col, dev, i32)
+    if O_row_ptr.device != dev or O_row_ptr.dtype != i32 or not O_row_ptr.is_contiguous():
+        _bad_operand("O_row_ptr", O_row_ptr, dev, i32)
+    if g.numel() != 8 * M:
+        raise RuntimeError(f"g must have {8 * M} elements")
+    if h.numel() != N:
+        raise RuntimeError(f"h must have {N} elements")
+    if O_row_ptr.numel() != M + 1:
+        raise RuntimeError(f"O_row_ptr must have {M + 1} elements")
+    if O_vals.numel() != 8 * O_col.numel():
+        raise RuntimeError("O_vals must be (nnz, 8) with nnz = len(O_col)")
+    if codes.device != dev or not codes.is_contiguous():
+        raise RuntimeError("codebook must be contiguous on the layer's device")
+    if codes.dtype != f16 and codes.dtype != torch.float32:
+        raise RuntimeError("codebook must be fp16 or fp32")
+    if codes.numel() != (2048 if kind == "e8_d4" else 524280):
+        raise RuntimeError(f"{kind} codebook must have {512 if kind == 'e8_d4' else 65535} rows")
     n_groups = 0
     if S_group is not None:
-        _require(S_group.device == dev and S_group.dtype == torch.float16 and S_group.is_contiguous(),
-                 "S_group must be a contiguous fp16 tensor on the layer's device")
-        _require(S_group.dim() == 2 and S_group.shape[1] == N, "S_group must be (n_groups, in_features)")
-        n_groups = int(S_group.shape[0])
+        if S_group.device != dev or S_group.dtype != f16 or not S_group.is_contiguous():
+            raise RuntimeError("S_group must be a contiguous fp16 tensor on the layer's device")
+        if S_group.dim() != 2 or S_group.shape[1] != N:
+            raise RuntimeError("S_group must be (n_groups, in_features)")
+        n_groups = S_group.shape[0]
     return M, N, n_groups
 
 
@@ -82,30 +118,33 @@ def linear_forward(kind: str, Q, codes, g, h, x, O_vals, O_col, O_row_ptr, bias=
     ``two_pass`` (what the module's ops pass): the two-pass prefill instead of
     the fused C-ABI kernel where it is preferred (``_two_pass_into``)."""
     M, N, n_groups = _check_layer(kind, Q, codes, g, h, O_vals, O_col, O_row_ptr, S_group)
-    _require(x.device == Q.device, "x must be on the layer's device")
-    _require(x.dim() == 2 and x.shape[1] == N, f"x must be (B, {N})")
-    _require(x.dtype in (torch.float16, torch.bfloat16), "x must be fp16 or bf16")
-    _require(x.is_contiguous(), "x must be contiguous")
+    dev, xdt = Q.device, x.dtype
+    if x.device != dev:
+        raise RuntimeError("x must be on the layer's device")
+    if x.dim() != 2 or x.shape[1] != N:
+        raise RuntimeError(f"x must be (B, {N})")
+    if xdt != torch.float16 and xdt != torch.bfloat16:
+        raise RuntimeError("x must be fp16 or bf16")
+    if not x.is_contiguous():
+        raise RuntimeError("x must be contiguous")
     if bias is not None and bias.numel() > 0:
-        _require(bias.device == Q.device and bias.dtype == torch.float16 and bias.numel() == 8 * M
+        _require(bias.device == dev and bias.dtype == torch.float16 and bias.numel() == 8 * M
                  and bias.is_contiguous(), "bias must be a contiguous fp16 (out_features,) tensor")
-    B = int(x.shape[0])
-    y = torch.empty((B, 8 * M), dtype=x.dtype, device=x.device)
+    B = x.shape[0]
+    y = torch.empty((B, 8 * M), dtype=xdt, device=dev)
     if B == 0:
         return y
     lib = _lib.load()
     if two_pass and B >= (TWO_PASS_MIN_TOKENS if kind == "e8_d4" else TWO_PASS_MIN_TOKENS_E8):
-        layer = dict(Q=Q, g=g, h=h, O_vals=O_vals, O_col=O_col, O_row_ptr=O_row_ptr, bias=bias, S_group=S_group)
-        arr = (_lib.EptqLayer * 1)(_layer_entry(layer, M, n_groups, 0))
-        if _two_pass_into(lib, arr, codes, x, y, kind, stream_workspace(x.device)):
+        arr = (_lib.EptqLayer * 1)(_layer_entry(Q, g, h, O_vals, O_col, O_row_ptr, bias, S_group, M, n_groups, 0))
+        if _two_pass_into(lib, arr, codes, x, y, kind, stream_workspace(dev)):
             return y
     fn = lib.eptq_e8d4_forward if kind == "e8_d4" else lib.eptq_e8_forward
-    with torch.cuda.device(x.device):
-        stream = torch.cuda.current_stream().cuda_stream
+    with _on(dev):
         rc = fn(_ptr(Q), _ptr(codes), EPTQ_F32 if codes.dtype == torch.float32 else EPTQ_F16,
-                _ptr(g), _ptr(h), _ptr(x), EPTQ_BF16 if x.dtype == torch.bfloat16 else EPTQ_F16,
+                _ptr(g), _ptr(h), x.data_ptr(), EPTQ_BF16 if xdt == torch.bfloat16 else EPTQ_F16,
                 _ptr(O_vals), _ptr(O_col), _ptr(O_row_ptr), _ptr(bias), _ptr(S_group), n_groups,
-                M, N, B, _ptr(y), stream)
+                M, N, B, y.data_ptr(), _raw_stream(dev))
     _lib.check(rc, fn.__name__)
     return y
 
@@ -138,11 +177,11 @@ def stream_workspace(device) -> Optional[torch.Tensor]:
     device = torch.device(device)
     if torch.cuda.is_current_stream_capturing():
         return None
-    stream = torch.cuda.current_stream(device)
-    key = (device.index if device.index is not None else torch.cuda.current_device(), stream.cuda_stream)
+    index = device.index if device.index is not None else torch.cuda.current_device()
+    key = (index, torch._C._cuda_getCurrentRawStream(index))
     w = _STREAM_WORK.get(key)
     if w is None:
-        w = _workspace_outside_graph_pools(device, stream)
+        w = _workspace_outside_graph_pools(device, torch.cuda.current_stream(device))
         _STREAM_WORK[key] = w
     return w
 
@@ -197,7 +236,7 @@ def _two_pass_into(lib, arr, codes, x, y, kind: str, work: Optional[torch.Tensor
     if B < (TWO_PASS_MIN_TOKENS if kind == "e8_d4" else TWO_PASS_MIN_TOKENS_E8) and not always:
         return False
     e8, xdt = int(kind != "e8_d4"), EPTQ_BF16 if x.dtype == torch.bfloat16 else EPTQ_F16
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         nbytes = lib.eptq_two_pass_scratch_bytes(e8, n, arr, N, B, xdt, int(work is not None), int(always))
         if nbytes == 0:
             return False
@@ -207,14 +246,14 @@ def _two_pass_into(lib, arr, codes, x, y, kind: str, work: Optional[torch.Tensor
         rc = lib.eptq_two_pass_forward(
             e8, n, arr, codes.data_ptr(), EPTQ_F32 if codes.dtype == torch.float32 else EPTQ_F16, x.data_ptr(), xdt, N,
             B, y.data_ptr(), y.shape[1], scratch.data_ptr(), nbytes, _ptr(work), 0 if work is None else work.numel(),
-            torch.cuda.current_stream().cuda_stream)
+            _raw_stream(x.device))
     _lib.check(rc, "eptq_two_pass_forward")
     return True
 
 
-def _layer_entry(L, M: int, n_groups: int, off: int):
-    return _lib.EptqLayer(_ptr(L["Q"]), _ptr(L["g"]), _ptr(L["h"]), _ptr(L["O_vals"]), _ptr(L["O_col"]),
-                          _ptr(L["O_row_ptr"]), _ptr(L.get("bias")), _ptr(L.get("S_group")), n_groups, M, off)
+def _layer_entry(Q, g, h, O_vals, O_col, O_row_ptr, bias, S_group, M: int, n_groups: int, off: int):
+    return _lib.EptqLayer(_ptr(Q), _ptr(g), _ptr(h), _ptr(O_vals), _ptr(O_col), _ptr(O_row_ptr), _ptr(bias),
+                          _ptr(S_group), n_groups, M, off)
 
 
 def linear_forward_multi(layers, codes, x, work: Optional[torch.Tensor] = None,
@@ -228,32 +267,38 @@ def linear_forward_multi(layers, codes, x, work: Optional[torch.Tensor] = None,
     ``decode_workspace`` (lets batches of 3..16 split the columns of layers
     with few row tiles over several workgroups); calls sharing one must not
     overlap in time."""
-    _require(len(layers) > 0, "no layers")
-    _require(x.dim() == 2 and x.dtype in (torch.float16, torch.bfloat16) and x.is_contiguous(),
-             "x must be a contiguous 2-D fp16/bf16 tensor")
-    N = int(x.shape[1])
+    return _forward_multi([(L["Q"], L["g"], L["h"], L["O_vals"], L["O_col"], L["O_row_ptr"], L.get("bias"),
+                            L.get("S_group")) for L in layers], codes, x, work, two_pass)
+
+
+def _forward_multi(layers, codes, x, work, two_pass) -> torch.Tensor:
+    """``linear_forward_multi`` on tuples (Q, g, h, O_vals, O_col, O_row_ptr, bias, S_group)."""
+    if len(layers) == 0:
+        raise RuntimeError("no layers")
+    xdt = x.dtype
+    if x.dim() != 2 or (xdt != torch.float16 and xdt != torch.bfloat16) or not x.is_contiguous():
+        raise RuntimeError("x must be a contiguous 2-D fp16/bf16 tensor")
+    B, N = x.shape
+    dev = x.device
     arr = (_lib.EptqLayer * len(layers))()
     off = 0
-    for i, L in enumerate(layers):
-        M, n2, n_groups = _check_layer("e8_d4", L["Q"], codes, L["g"], L["h"], L["O_vals"], L["O_col"],
-                                       L["O_row_ptr"], L.get("S_group"))
-        _require(n2 == N and L["Q"].device == x.device, "layers must take x's in_features on x's device")
-        arr[i] = _layer_entry(L, M, n_groups, off)
+    for i, (Q, g, h, O_vals, O_col, O_row_ptr, bias, S_group) in enumerate(layers):
+        M, n2, n_groups = _check_layer("e8_d4", Q, codes, g, h, O_vals, O_col, O_row_ptr, S_group)
+        if n2 != N or Q.device != dev:
+            raise RuntimeError("layers must take x's in_features on x's device")
+        arr[i] = _layer_entry(Q, g, h, O_vals, O_col, O_row_ptr, bias, S_group, M, n_groups, off)
         off += 8 * M
-    B = int(x.shape[0])
-    y = torch.empty((B, off), dtype=x.dtype, device=x.device)
+    y = torch.empty((B, off), dtype=xdt, device=dev)
     if B == 0:
         return y
     lib = _lib.load()
-    if two_pass and _two_pass_into(lib, arr, codes, x, y, "e8_d4", work):
+    if two_pass and B >= TWO_PASS_MIN_TOKENS and _two_pass_into(lib, arr, codes, x, y, "e8_d4", work):
         return y
-    with torch.cuda.device(x.device):
-        stream = torch.cuda.current_stream().cuda_stream
-        rc = lib.eptq_e8d4_forward_multi(len(layers), arr, _ptr(codes),
-                                         EPTQ_F32 if codes.dtype == torch.float32 else EPTQ_F16, _ptr(x),
-                                         EPTQ_BF16 if x.dtype == torch.bfloat16 else EPTQ_F16, N, B,
-                                         _ptr(y), off, _ptr(work), 0 if work is None else work.numel(),
-                                         stream)
+    with _on(dev):
+        rc = lib.eptq_e8d4_forward_multi(len(layers), arr, codes.data_ptr(),
+                                         EPTQ_F32 if codes.dtype == torch.float32 else EPTQ_F16, x.data_ptr(),
+                                         EPTQ_BF16 if xdt == torch.bfloat16 else EPTQ_F16, N, B, y.data_ptr(), off,
+                                         _ptr(work), 0 if work is None else work.numel(), _raw_stream(dev))
     _lib.check(rc, "eptq_e8d4_forward_multi")
     return y
 
@@ -272,10 +317,9 @@ def dequant(kind: str, Q, codes, g, h, O_vals, O_col, O_row_ptr, S_group=None,
         W = out
     lib = _lib.load()
     fn = lib.eptq_e8d4_dequant if kind == "e8_d4" else lib.eptq_e8_dequant
-    with torch.cuda.device(Q.device):
-        stream = torch.cuda.current_stream().cuda_stream
+    with _on(Q.device):
         rc = fn(_ptr(Q), _ptr(codes), _ptr(g), _ptr(h), _ptr(O_vals), _ptr(O_col),
-                _ptr(O_row_ptr), _ptr(S_group), n_groups, M, N, _ptr(W), stream)
+                _ptr(O_row_ptr), _ptr(S_group), n_groups, M, N, _ptr(W), _raw_stream(Q.device))
     _lib.check(rc, fn.__name__)
     return W
 
@@ -292,9 +336,8 @@ def f16_gemm(W: torch.Tensor, x: torch.Tensor, bias: Optional[torch.Tensor] = No
     F, N = int(W.shape[0]), int(W.shape[1])
     T = int(x.shape[0])
     y = torch.empty((T, F), dtype=torch.float16, device=x.device)
-    with torch.cuda.device(x.device):
-        rc = _lib.load().eptq_f16_gemm(_ptr(W), _ptr(x), _ptr(bias), F, N, T, _ptr(y), F,
-                                       torch.cuda.current_stream().cuda_stream)
+    with _on(x.device):
+        rc = _lib.load().eptq_f16_gemm(_ptr(W), _ptr(x), _ptr(bias), F, N, T, _ptr(y), F, _raw_stream(x.device))
     _lib.check(rc, "eptq_f16_gemm")
     return y
 
@@ -394,11 +437,12 @@ def e8d4_forward_multi(Q: List[torch.Tensor], codes: torch.Tensor, g: List[torch
     (declared mutated: the split-K parts write their partial sums there; the
     counters return to zero), or None for the current stream's own (``stream_workspace``), which the op
     looks up when it runs, like a BLAS library's internal workspace."""
-    layers = [dict(Q=Q[i], g=g[i], h=h[i], O_vals=O_vals[i], O_col=O_col[i], O_row_ptr=O_row_ptr[i],
-                   bias=bias[i], S_group=S_group[i]) for i in range(len(Q))]
     if work is None and x.is_cuda:
         work = stream_workspace(x.device)
-    return linear_forward_multi(layers, codes, x, work=work, two_pass=True)
+    n = len(Q)
+    if any(len(t) < n for t in (g, h, O_vals, O_col, O_row_ptr, bias, S_group)):
+        raise IndexError("list index out of range")
+    return _forward_multi(list(zip(Q, g, h, O_vals, O_col, O_row_ptr, bias, S_group)), codes, x, work, True)
 
 
 @e8d4_forward_multi.register_fake

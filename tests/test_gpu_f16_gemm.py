@@ -144,8 +144,8 @@ def test_two_pass_split_and_together(outs, inp, T, dt, qb):
     arr = (_lib.EptqLayer * len(lins))()
     off = 0
     for k, l in enumerate(lins):
-        L = {n: getattr(l, n) for n in ("Q", "g", "h", "O_vals", "O_col", "O_row_ptr", "bias", "S_group")}
-        arr[k] = _layer_entry(L, outs[k] // 8, 0 if qb is None else outs[k] // qb, off)
+        arr[k] = _layer_entry(*(getattr(l, n) for n in ("Q", "g", "h", "O_vals", "O_col", "O_row_ptr", "bias", "S_group")),
+                              outs[k] // 8, 0 if qb is None else outs[k] // qb, off)
         off += outs[k]
     want = torch.cat([x.float() @ l.dequantize().float().t() + (l.bias.float() if l.bias is not None else 0)
                       for l in lins], dim=-1)
