@@ -13,7 +13,8 @@ from pathlib import Path
 
 ROOT = Path(__file__).resolve().parent
 REPO = ROOT.parent
-SOURCES = ["abi.hip", "dequant.hip", "matvec.hip", "decode.hip", "decode_mfma.hip", "decode_wide.hip", "gemm.hip", "llama_ops.hip"]
+SOURCES = ["abi.hip", "dequant.hip", "matvec.hip", "decode.hip", "decode_mfma.hip", "decode_wide.hip", "gemm.hip", "llama_ops.hip",
+           "llama_prompt.hip"]
 OUT = ROOT / "_lib" / "libeptq_hip.so"
 
 HIPCC_FLAGS = [

@@ -47,6 +47,7 @@ _F = ctypes.c_float
 LLAMA_SIGNATURES = {
     "eptq_llama_rmsnorm": ([_P, _P, _P, _P, _I, _I, _F, _P], _I),
     "eptq_llama_rope_attn": ([_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _P], _I),
+    "eptq_llama_prompt_attn": ([_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P], _I),
     "eptq_llama_attn_work_bytes": ([_I, _I], ctypes.c_longlong),
     "eptq_llama_silu_mul": ([_P, _P, _I, _I, _P], _I),
     "eptq_llama_norm_linear": ([_I, _P, _P, _P, _P, _P, _F, _P, _I, _I, _P, _I, _P], _I),

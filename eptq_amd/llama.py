@@ -14,7 +14,9 @@ and silu(gate)·up at its output -> down, the residual adds inside the o and
 down launches (B <= 2: inside the q|k|v and gate|up launches).  Shapes are
 static (preallocated cache, position in a device tensor), so the step is
 captured once in a HIP graph and replayed.
-Prefill (many tokens) runs the same Linears (MFMA GEMM) and PyTorch attention.
+Prefill (many tokens) runs the same Linears (MFMA GEMM), the RMSNorm and SwiGLU
+kernels and one attention kernel with rotary and cache writes; PyTorch operators
+where head_dim is not 128 or ``fused_ops`` is off.
 Greedy decoding.
 """
 
@@ -188,7 +190,7 @@ class DecoderLayer(nn.Module):
         self.down_proj = lin["down_proj"]
 
     def forward(self, x, cos, sin, kc, vc, pos, mask):
-        """Prefill (T tokens): x (B, T, hidden); caches (B, Hkv, L, D); pos (T,)
+        """Prefill (T tokens) on PyTorch operators: x (B, T, hidden); caches (B, Hkv, L, D); pos (T,)
         positions; mask (T, L) additive.  PyTorch attention."""
         cfg = self.cfg
         B, T, _ = x.shape
@@ -214,6 +216,23 @@ class DecoderLayer(nn.Module):
         gu = self.gate_up_proj(h).float()
         a = F.silu(gu[..., :cfg.ffn]) * gu[..., cfg.ffn:]
         return x + self.down_proj(a.to(x.dtype))
+
+    def prompt(self, x, delta, cos_tab, sin_tab, kc, vc, pos, T):
+        """The same on the HIP kernels: x (B·T, hidden) the residual stream, updated
+        in place (x += delta first, the previous layer's output); returns this
+        layer's output, the delta of the next.  The norms take the residual adds
+        with them, and rotary, cache writes and attention are
+        ``eptq_llama_prompt_attn``."""
+        cfg = self.cfg
+        rows = x.shape[0]
+        qkv = self.qkv_proj(rmsnorm_(x, delta, self.input_layernorm.weight, cfg.eps))
+        att = torch.empty((rows, cfg.heads * cfg.head_dim), dtype=x.dtype, device=x.device)
+        rc = _lib.load().eptq_llama_prompt_attn(
+            qkv.data_ptr(), pos.data_ptr(), cos_tab.data_ptr(), sin_tab.data_ptr(), kc.data_ptr(), vc.data_ptr(),
+            att.data_ptr(), rows // T, T, cfg.heads, cfg.kv_heads, cfg.head_dim, kc.shape[2], _stream(x))
+        _lib.check(rc, "eptq_llama_prompt_attn")
+        h = rmsnorm_(x, self.o_proj(att), self.post_attention_layernorm.weight, cfg.eps)
+        return self.down_proj(silu_mul(self.gate_up_proj(h)))
 
 
 class QuantLlama(nn.Module):
@@ -265,8 +284,27 @@ class QuantLlama(nn.Module):
 
     def forward_tokens(self, ids, pos):
         """ids: (B, T) int64, pos: (T,) int64 positions -> logits (B, T, vocab)."""
+        return self._forward_tokens(ids, pos, self.fused_ops)
+
+    def _hip_prompt(self, x, ids, pos):
+        """Whether the HIP prompt kernels take this call (else PyTorch operators):
+        a whole fp16 model without gradients, head_dim 128."""
+        cfg = self.cfg
+        w = self.norm.weight
+        return (cfg.head_dim == 128 and cfg.hidden % 8 == 0 and cfg.hidden <= 16384 and cfg.ffn % 8 == 0
+                and cfg.heads % cfg.kv_heads == 0 and x.is_cuda and x.dtype == torch.float16
+                and w.dtype == torch.float16 and self.kc[0].dtype == torch.float16
+                and pos.dtype == torch.int64 and pos.is_contiguous() and pos.shape == (ids.shape[1],)
+                and pos.device == x.device and 0 < ids.numel() <= 65535 and not (torch.is_grad_enabled() and x.requires_grad))
+
+    def _forward_tokens(self, ids, pos, fused):
         x = self.embed_tokens(ids)
         T = ids.shape[1]
+        if fused and self._hip_prompt(x, ids, pos):
+            r, delta = x.reshape(-1, self.cfg.hidden), None
+            for i, layer in enumerate(self.layers):
+                delta = layer.prompt(r, delta, self.cos_tab, self.sin_tab, self.kc[i], self.vc[i], pos, T)
+            return self.lm_head(rmsnorm_(r, delta, self.norm.weight, self.cfg.eps).reshape(x.shape))
         cos = self.cos_tab.index_select(0, pos)[None, None]
         sin = self.sin_tab.index_select(0, pos)[None, None]
         L = self.max_len
@@ -463,8 +501,8 @@ class GraphDecoder:
     """Greedy decode with the per-token step captured in a HIP graph.
 
     ``fused=True`` runs the step on the fused decode kernels
-    (``QuantLlama.decode_tokens``); ``fused=False`` on the PyTorch-attention
-    path used for prefill (``forward_tokens``), kept as a cross-check."""
+    (``QuantLlama.decode_tokens``); ``fused=False`` on PyTorch operators around
+    the same Linears, kept as a cross-check."""
 
     def __init__(self, model: QuantLlama, batch: int, max_len: int, device="cuda", fused: bool = True):
         self.model = model
@@ -494,7 +532,7 @@ class GraphDecoder:
         self._check_owner()
         T = prompt.shape[1]
         pos = torch.arange(T, device=self.device)
-        logits = self.model.forward_tokens(prompt, pos)
+        logits = self.model._forward_tokens(prompt, pos, self.fused and self.model.fused_ops)
         nxt = logits[:, -1].argmax(-1, keepdim=True)
         self.tok.copy_(nxt)
         self.pos.fill_(T)
@@ -505,7 +543,7 @@ class GraphDecoder:
         if self.fused:
             self.model.decode_next(self.tok, self.pos)
         else:
-            logits = self.model.forward_tokens(self.tok, self.pos)[:, -1]
+            logits = self.model._forward_tokens(self.tok, self.pos, False)[:, -1]
             self.tok.copy_(logits.argmax(-1, keepdim=True))
             self.pos.add_(1)
 

@@ -38,6 +38,17 @@ int eptq_llama_rope_attn(const void* qkv, const void* pos, const void* cos_tab, 
                          void* k_cache, void* v_cache, void* out, int B, int H, int Hk, int D, int L,
                          void* work, void* stream);
 
+/* Attention of T tokens per sequence at positions pos[0..T) (int64 on the
+ * device, each below L): rotary on q and k, k and v written to the caches
+ * (B, Hk, L, D) at their positions, out (B·T, H·D) = softmax(q·Kᵀ/√D)·V over
+ * the cache rows 0..pos[t] of each token.  qkv is (B·T, (H + 2 Hk)·D) as
+ * above, row b·T + t.  A token whose position lies outside the cache writes
+ * nothing to it and has no defined output.  D == 128 (2 otherwise), H % Hk ==
+ * 0, pointers 16-byte aligned. */
+int eptq_llama_prompt_attn(const void* qkv, const void* pos, const void* cos_tab, const void* sin_tab,
+                           void* k_cache, void* v_cache, void* out, int B, int T, int H, int Hk, int D, int L,
+                           void* stream);
+
 /* Bytes of the eptq_llama_rope_attn workspace for B batch rows and H heads. */
 long long eptq_llama_attn_work_bytes(int B, int H);
 
