@@ -288,14 +288,19 @@ class QuantLlama(nn.Module):
 
     def _hip_prompt(self, x, ids, pos):
         """Whether the HIP prompt kernels take this call (else PyTorch operators):
-        a whole fp16 model without gradients, head_dim 128."""
+        a whole fp16 model without gradients, head_dim 128, one sequence per
+        cache row (the kernel addresses the caches by sequence, so any other
+        batch or a prompt longer than the cache stays with the operators'
+        own checks)."""
         cfg = self.cfg
         w = self.norm.weight
         return (cfg.head_dim == 128 and cfg.hidden % 8 == 0 and cfg.hidden <= 16384 and cfg.ffn % 8 == 0
                 and cfg.heads % cfg.kv_heads == 0 and x.is_cuda and x.dtype == torch.float16
                 and w.dtype == torch.float16 and self.kc[0].dtype == torch.float16
                 and pos.dtype == torch.int64 and pos.is_contiguous() and pos.shape == (ids.shape[1],)
-                and pos.device == x.device and 0 < ids.numel() <= 65535 and not (torch.is_grad_enabled() and x.requires_grad))
+                and pos.device == x.device and 0 < ids.numel() <= 65535
+                and ids.shape[0] == self.kc[0].shape[0] and ids.shape[1] <= self.max_len
+                and not (torch.is_grad_enabled() and any(p.requires_grad for p in self.parameters())))
 
     def _forward_tokens(self, ids, pos, fused):
         x = self.embed_tokens(ids)

@@ -69,3 +69,24 @@ def test_prompt_attention_rejects_other_head_dims():
     x = torch.zeros(64, dtype=torch.float16, device="cuda")
     rc = _lib.load().eptq_llama_prompt_attn(*([x.data_ptr()] * 7), 1, 1, 1, 1, 64, 1, 0)
     assert rc == 2
+
+
+def test_prompt_kernels_only_for_the_caches_batch_and_length():
+    """The kernel addresses the caches by sequence: other batches keep the refusal of the PyTorch operators, and a
+    prompt longer than the cache and a model with trainable parameters never reach it."""
+    from eptq_amd.llama import LlamaConfig, build_synthetic
+    model = build_synthetic(LlamaConfig(hidden=256, ffn=256, layers=1, heads=2, kv_heads=2, vocab=64), device="cuda", seed=3)
+    model.alloc_cache(1, 8, "cuda")
+
+    def taken(B, T):
+        ids = torch.zeros((B, T), dtype=torch.int64, device="cuda")
+        return model._hip_prompt(model.embed_tokens(ids), ids, torch.arange(T, device="cuda"))
+
+    assert taken(1, 1) and taken(1, 8)
+    assert not taken(1, 9) and not taken(2, 8)
+    model.norm.weight.requires_grad_(True)
+    assert not taken(1, 8)
+    with torch.no_grad():
+        assert taken(1, 8)
+        with pytest.raises((RuntimeError, IndexError)):
+            model.forward_tokens(torch.zeros((2, 4), dtype=torch.int64, device="cuda"), torch.arange(4, device="cuda"))
