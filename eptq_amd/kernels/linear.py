@@ -17,8 +17,8 @@ Differences, all towards the reference's own reconstruct semantics:
 * every batch size runs a hand-written HIP kernel of this library: the decode
   matvec for ≤16 rows, the wide matrix-core decode (E8-D4) up to 128 rows,
   the prefill GEMM that decodes weight tiles into LDS above (the reference's
-  ``csrc/eptq_kernels.cu:520-537`` route), and from 2048 fp16 tokens (256
-  for S_group layers or bf16 x, 64 for E8 layers) the two-pass prefill: each weight
+  ``csrc/eptq_kernels.cu:520-537`` route), and where it is estimated faster
+  (S_group layers or bf16 x: from 129 rows, E8 layers: from 17) the two-pass prefill: each weight
   decoded once into a transient fp16 W (freed on return), then this
   library's W-streaming GEMM.  No library GEMM runs.  ``EPTQ_CUDA_DECODE`` / ``EPTQ_FORCE_TRITON`` are
   accepted and ignored.
